@@ -15,7 +15,7 @@
 //
 // Two kernels: a streaming one for T <= 64 (weights read once, the
 // routing-weighted combine fused in) and an LDS-tiled one for larger T (fp32
-// rows to the combine pass).
+// rows to the combine pass), with tiles of their own for experts of few rows.
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -386,14 +386,222 @@ struct G2Tiled {
   static constexpr int kGroupM = 4;
 };
 
-template <int WM, int WN, int MI, int NJ, int STAGES>
+// ---------------------------------------------------------------------------
+// Low tiles: experts of at most 32 rows (one row tile, so W2 is read once).
+//
+// Bound by the W2 stream.  The 64 x 256 tile above reads it in 64-K steps,
+// half of each 128-byte line at a time: a read-only probe of that pattern (672
+// tiles, 352 MB) reaches 4.6 TB/s against 5.1 with whole lines and 5.7 with
+// whole lines and nontemporal copies (with half lines nt fetches them twice,
+// 3.5), and the step's barrier makes every wave wait for the slowest of all
+// copies.  Here
+//   * each wave owns 32 output columns and copies their W2 rows itself, 128 K
+//     (one scale block, whole lines, nt) at a time, into two slots of its own
+//     LDS: no barrier stands between a W2 copy and its use, and a slot is
+//     refilled as soon as its fragments are in registers, so two K blocks
+//     stay in flight (64 KB of W2 per workgroup, two workgroups per CU);
+//   * the act rows are shared: one plane per wave and stage.  RB = 1 (16
+//     rows) stages 128 K, the next stage's copy issued before the W2 copy of
+//     two blocks ahead (the vector-memory counter completes in order: a wait
+//     for act rows issued after it would wait for that W2 too).  RB = 2 (32
+//     rows) stages 64 K and holds a stage in registers, a second barrier
+//     freeing its slot at once for the stage two ahead;
+//   * e4m3 -> bf16 conversions run once per W2 value (the 64 x 256 tile's two
+//     row waves each convert all of a column's).
+// Interleaved A/B, GEMM2 us (64 x 256 tiles only -> with low tiles): prefill
+// routing T = 65 48 -> 40, 333 102 -> 79, 512 97 -> 76, 700 104 -> 93, 1024
+// 107 -> 102, 2000 150 -> 148, 3000 195 -> 193; hot experts T = 128 80 -> 65,
+// 1451 335 -> 328.  An extra row block (33 to 64 rows, act rows 32 KB per 128
+// K) gained nothing, nor did 48-column waves; low tiles ahead of the others
+// lost 5-8 us at T = 128 to 512 (they are the shorter ones).
+// ---------------------------------------------------------------------------
+template <int RB_>
+struct G2Low {
+  static constexpr int RB = RB_;                 // 16-row blocks
+  static constexpr int BM = 16 * RB;
+  static constexpr int NF = 2;                   // 16-column blocks per wave
+  static constexpr int kWaves = 8;
+  static constexpr int kWaveCols = 16 * NF;
+  static constexpr int BN = kWaveCols * kWaves;
+  static constexpr int kNT = kH / BN;
+  static_assert(kH % BN == 0 && kBlk % kWaveCols == 0, "column tiles; a wave's columns lie in one scale block");
+  static constexpr int kFrag = 2048;             // 16 W2 rows x 128 K
+  static constexpr int kWSlot = NF * kFrag;
+  static constexpr int kWOps = 2 * NF;           // copies per wave of one K block
+  static constexpr int D = 2;                    // W2 slots per wave
+  static constexpr int kAFrag = 4096;            // 16 act rows x 64 K: hi (two wide planes), lo (two)
+  static constexpr int KH = RB == 1 ? 2 : 1;     // half steps (64 K) per A stage
+  static constexpr int kAStage = RB * KH * kAFrag;
+  static_assert(RB * KH * 4 == kWaves, "one A plane per wave and stage");
+  static constexpr int kAOff = kWaves * D * kWSlot;
+  static constexpr int kLdsBytes = kAOff + 2 * kAStage;
+};
+
+template <class C>
+__device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __restrict__ act,
+                                               const uint8_t* __restrict__ w2, const float* __restrict__ w2_scale,
+                                               float* __restrict__ down, int e, int row0, int rows, int n0) {
+  constexpr int RB = C::RB, NF = C::NF, D = C::D, KH = C::KH;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lane = threadIdx.x & (kWave - 1);
+  const int lq = lane >> 4;
+  const int lr = lane & 15;
+  const int nw = n0 + C::kWaveCols * wave;  // the wave's first column
+  const char* wbase = (const char*)(w2 + ((size_t)e * kH + nw) * kI);
+  const char* abase = (const char*)(act + (size_t)row0 * kActRowElems);
+  char* wring = lds + wave * (D * C::kWSlot);
+  char* aring = lds + C::kAOff;
+  uint32_t woff[2];  // column block 0, rows 0-7 / 8-15
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    int m, chunk;
+    wide_copy_lane(lane, h, m, chunk);
+    woff[h] = (uint32_t)m * kI + 16 * chunk;
+  }
+  uint32_t aoff;
+  {
+    const int f = wave >> 2, h = (wave >> 1) & 1;  // ((half step, row block), hi / lo, rows 0-7 / 8-15)
+    int fr, chunk;
+    wide_copy_lane(lane, wave & 1, fr, chunk);
+    const int r = min((f % RB) * 16 + fr, rows - 1);
+    aoff = (uint32_t)r * (kActRowElems * 2) + (f / RB) * 256 + 128 * h + 16 * chunk;
+  }
+  auto issue_w = [&](int kb) {
+    uint32_t ko = kb * kBlk;
+    asm volatile("" : "+s"(ko));  // added at use: no strength-reduced copies of the offsets
+    char* wslot = wring + (kb % D) * C::kWSlot;
+#pragma unroll
+    for (int c = 0; c < NF; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) dma16_nt(wbase + (uint32_t)(woff[h] + (ko + c * 16 * kI)), wslot + c * C::kFrag + h * 1024);
+  };
+  auto issue_a = [&](int j) {
+    uint32_t jo = j * KH * 256;
+    asm volatile("" : "+s"(jo));
+    dma16(abase + (uint32_t)(aoff + jo), aring + (j & 1) * C::kAStage + wave * 1024);
+  };
+  const float sv = w2_scale[((size_t)e * kNHBlk + nw / kBlk) * kNIBlk + lr];  // scale of K block lr
+  const int slot_a0 = wide_slot(lr, 2 * lq), slot_a1 = wide_slot(lr, 2 * lq + 1);
+  const int slot_b0 = wide_slot(lr, lq), slot_b1 = wide_slot(lr, 4 + lq);
+
+  v4f acc[RB][NF], P[RB][NF];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int c = 0; c < NF; ++c) acc[rb][c] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  v4i raw[NF][2];
+  issue_a(0);
+  issue_w(0);
+  if (D == 2) issue_w(1);
+  if (RB == 2) issue_a(1);
+  // Half step h = 2 kb + g of 64 K; LEFT: K blocks after this one (2: at least
+  // two).  Each wait leaves what was issued after the half step's operands:
+  // RB = 1: W(kb + 1); RB = 2: g = 0 W(kb + 1), A(h + 1); g = 1 A(h + 1), W(kb + 2).
+  auto half = [&](int kb, auto g_c, auto left_c) {
+    constexpr int g = decltype(g_c)::value, LEFT = decltype(left_c)::value;
+    const int h = 2 * kb + g;
+    if constexpr (RB == 1) {
+      if (g == 0) {
+        wait_vmcnt_lgkm0<D == 2 && LEFT >= 1 ? C::kWOps : 0>();
+        block_barrier();
+        if (LEFT >= 1) issue_a(kb + 1);
+      }
+    } else {
+      wait_vmcnt_lgkm0<g == 0 ? (D == 2 && LEFT >= 1 ? C::kWOps : 0) + 1
+                              : (LEFT >= D ? C::kWOps : 0) + (LEFT >= 1 ? 1 : 0)>();
+      block_barrier();
+    }
+    if (g == 0) {
+      const char* wslot = wring + (kb % D) * C::kWSlot;
+#pragma unroll
+      for (int c = 0; c < NF; ++c) {
+        raw[c][0] = *(const v4i*)(wslot + c * C::kFrag + slot_b0);
+        raw[c][1] = *(const v4i*)(wslot + c * C::kFrag + slot_b1);
+      }
+    }
+    const char* ab = aring + ((KH == 2 ? kb : h) & 1) * C::kAStage + (KH == 2 ? g * C::kAFrag : 0);
+    v8bf a[RB][4];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const char* f = ab + rb * C::kAFrag;
+      a[rb][0] = *(const v8bf*)(f + slot_a0);
+      a[rb][1] = *(const v8bf*)(f + slot_a1);
+      a[rb][2] = *(const v8bf*)(f + 2048 + slot_a0);
+      a[rb][3] = *(const v8bf*)(f + 2048 + slot_a1);
+    }
+    if constexpr (RB == 2) {
+      // the half step's rows go to registers: their slot takes half step h + 2
+      lds_barrier();
+      if (LEFT >= 1) issue_a(h + 2);
+    } else if (g == 0) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the W2 slot is read: free for block kb + 2
+    }
+    if (g == 0 && LEFT >= D) issue_w(kb + D);
+#pragma unroll
+    for (int c = 0; c < NF; ++c) {
+      const v8bf b0 = e4m3x8_to_bf16((uint32_t)raw[c][g][0], (uint32_t)raw[c][g][1]);
+      const v8bf b1 = e4m3x8_to_bf16((uint32_t)raw[c][g][2], (uint32_t)raw[c][g][3]);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        P[rb][c] = mfma_bf16_16x16x32(b0, a[rb][0], g == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : P[rb][c]);
+        P[rb][c] = mfma_bf16_16x16x32(b1, a[rb][1], P[rb][c]);
+        P[rb][c] = mfma_bf16_16x16x32(b0, a[rb][2], P[rb][c]);
+        P[rb][c] = mfma_bf16_16x16x32(b1, a[rb][3], P[rb][c]);
+      }
+    }
+    if (g == 1) {
+      const float sb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sv), kb));
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int c = 0; c < NF; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[rb][c][i] = __builtin_fmaf(P[rb][c][i], sb, acc[rb][c][i]);
+    }
+  };
+  auto block = [&](int kb, auto left_c) {
+    half(kb, std::integral_constant<int, 0>{}, left_c);
+    half(kb, std::integral_constant<int, 1>{}, left_c);
+  };
+#pragma unroll 1
+  for (int kb = 0; kb < kNIBlk - 2; ++kb) block(kb, std::integral_constant<int, 2>{});
+  __builtin_amdgcn_sched_barrier(0);
+  block(kNIBlk - 2, std::integral_constant<int, 1>{});
+  __builtin_amdgcn_sched_barrier(0);
+  block(kNIBlk - 1, std::integral_constant<int, 0>{});
+  __builtin_amdgcn_sched_barrier(0);
+  // lane (q, r): row r, columns 4q .. 4q + 3 of each 16
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int r = rb * 16 + lr;
+    if (r < rows) {
+#pragma unroll
+      for (int c = 0; c < NF; ++c)
+        *(v4f*)(down + (size_t)(row0 + r) * kH + nw + 16 * c + 4 * lq) = acc[rb][c];
+    }
+  }
+}
+
+// Low tiles up to this T.  T = 3000 gains 1 % of GEMM2, T = 4096 ties (255 / 252
+// us); at T = 8192 and 14107 (uniform routing, many rounds of full tiles) the
+// few low tiles at the end of the launch run alone, bound by latency: 405 ->
+// 407, 746 -> 758 us.
+constexpr int kG2LowMaxTokens = 3072;
+
+// LOW: with low tiles (a kernel of its own: the full tiles ran 1 % slower
+// beside their code at T = 14107).
+template <int WM, int WN, int MI, int NJ, int STAGES, bool LOW>
 __global__ void __launch_bounds__(64 * WM * WN, 4)
 gemm2_tiled_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__ w2,
                    const float* __restrict__ w2_scale, const int32_t* __restrict__ expert_off,
                    float* __restrict__ down, int T) {
   using C = G2Tiled<WM, WN, MI, NJ, STAGES>;
   // One LDS object (see gemm1.hip): the stage ring, then the weight scales.
-  __shared__ __attribute__((aligned(1024))) char lds[C::kStages * C::kStageBytes + C::kWscBytes];
+  constexpr int kFullLds = C::kStages * C::kStageBytes + C::kWscBytes;
+  constexpr int kLds = LOW && G2Low<2>::kLdsBytes > kFullLds ? G2Low<2>::kLdsBytes : kFullLds;
+  static_assert(G2Low<1>::kLdsBytes == G2Low<2>::kLdsBytes && 2 * kLds <= 160 * 1024, "two workgroups per CU");
+  __shared__ __attribute__((aligned(1024))) char lds[kLds];
 
   ExpertRows X;
   X.load(expert_off);
@@ -402,26 +610,30 @@ gemm2_tiled_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__
   // expert order into one accumulator (GEMM1 folded the routing weights into
   // their rows) and writes the sum to the first one's rows.
   const uint32_t fused = every_token_experts(X, T);
+  // Low experts (at most 32 rows) take low tiles (gemm2_low_tile).
+  const int lane_e = threadIdx.x & (kWave - 1);
+  const uint32_t low =
+      LOW ? (uint32_t)__ballot(lane_e < kELocal && X.cnt > 0 && X.cnt <= G2Low<2>::BM) & ~fused : 0u;
   int mt, nt, e, row0, rows;
   uint32_t tile_exps;  // the experts whose K loops this tile runs, in order
-  if (!fused) {
-    const int mt_total = X.count_tiles(C::BM);
-    const int t = xcd_tile(blockIdx.x, mt_total * C::kNT);
+  if (!(fused | low)) {
+    const int t = xcd_tile(blockIdx.x, X.count_tiles(C::BM) * C::kNT);
     if (t < 0) return;
     grouped_tile(X, t, C::BM, C::kNT, C::kGroupM, mt, nt);
     X.find_tile(mt, C::BM, e, row0, rows);
     tile_exps = 1u << e;
   } else {
-    // XCD x = block % 8 takes the x-th eighth of the fused tiles (the long
-    // ones) first, then the x-th eighth of the other experts' tiles.
-    const int lane = threadIdx.x & (kWave - 1);
-    ExpertRows Xs = X;
-    if (lane < kELocal && ((fused >> lane) & 1u)) Xs.cnt = 0;
-    const int frt = (T + C::BM - 1) / C::BM;  // fused row tiles
-    const int nf = frt * C::kNT, ns = Xs.count_tiles(C::BM) * C::kNT;
-    const int x = blockIdx.x % 8, l = blockIdx.x / 8;
+    // XCD x = block % 8 takes the x-th eighth of the fused tiles (the longest)
+    // first, then the x-th eighth of the full tiles, then of the low ones.
+    ExpertRows Xs = X;  // the experts of the full tiles
+    if (lane_e < kELocal && (((fused | low) >> lane_e) & 1u)) Xs.cnt = 0;
+    const int frt = fused ? (T + C::BM - 1) / C::BM : 0;  // fused row tiles
+    const int nf = frt * C::kNT, ns = Xs.count_tiles(C::BM) * C::kNT, nl = __builtin_popcount(low) * G2Low<1>::kNT;
+    const int x = blockIdx.x % 8;
     const int f0 = (int)((int64_t)x * nf / 8), f1 = (int)((int64_t)(x + 1) * nf / 8);
     const int s0 = (int)((int64_t)x * ns / 8), s1 = (int)((int64_t)(x + 1) * ns / 8);
+    const int l0 = (int)((int64_t)x * nl / 8), l1 = (int)((int64_t)(x + 1) * nl / 8);
+    const int l = blockIdx.x / 8;
     if (l < f1 - f0) {
       // L2 groups of kGroupM row tiles sweeping the column tiles, row tile fastest
       const int idx = f0 + l, per_group = C::kGroupM * C::kNT;
@@ -438,7 +650,19 @@ gemm2_tiled_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__
       Xs.find_tile(mt, C::BM, e, row0, rows);
       tile_exps = 1u << e;
     } else {
-      return;
+      const int t = l0 + l - (f1 - f0) - (s1 - s0);
+      if (!LOW || t >= l1) return;
+      if constexpr (LOW) {
+        e = nth_set_bit(low, t / G2Low<1>::kNT);
+        row0 = X.begin(e);
+        rows = X.end(e) - row0;
+        const int n0 = t % G2Low<1>::kNT * G2Low<1>::BN;
+        if (rows <= G2Low<1>::BM)
+          gemm2_low_tile<G2Low<1>>(lds, act, w2, w2_scale, down, e, row0, rows, n0);
+        else
+          gemm2_low_tile<G2Low<2>>(lds, act, w2, w2_scale, down, e, row0, rows, n0);
+        return;
+      }
     }
   }
   const int n_steps = __builtin_popcount(tile_exps) * C::kSteps;
@@ -608,14 +832,14 @@ gemm2_tiled_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__
       }
 }
 
-template <int WM, int WN, int MI, int NJ, int STAGES>
+template <bool LOW>
 hipError_t launch_gemm2_tiled(int T, const uint8_t* w2, const float* w2_scale, const Layout& L, char* ws,
                               hipStream_t stream) {
-  using C = G2Tiled<WM, WN, MI, NJ, STAGES>;
+  using C = G2Tiled<2, 4, 2, 4, 2>;
   const int64_t pairs = (int64_t)T * kTopK;
   const int64_t mtiles = (pairs + C::BM - 1) / C::BM + (pairs < kELocal ? pairs : kELocal);
   const int64_t blocks = ((mtiles * C::kNT + 7) / 8) * 8;
-  hipLaunchKernelGGL((gemm2_tiled_kernel<WM, WN, MI, NJ, STAGES>), dim3((unsigned)blocks), dim3(C::kThreads), 0,
+  hipLaunchKernelGGL((gemm2_tiled_kernel<2, 4, 2, 4, 2, LOW>), dim3((unsigned)blocks), dim3(C::kThreads), 0,
                      stream, (const uint16_t*)(ws + L.act), w2, w2_scale,
                      (const int32_t*)(ws + L.expert_off), (float*)(ws + L.down), T);
   return hipGetLastError();
@@ -633,7 +857,8 @@ hipError_t launch_gemm2(int T, const uint8_t* w2, const float* w2_scale, const L
                        (const int32_t*)(ws + L.perm_token), (const float*)(ws + L.perm_w), T, (uint16_t*)out);
     return hipGetLastError();
   }
-  return launch_gemm2_tiled<2, 4, 2, 4, 2>(T, w2, w2_scale, L, ws, stream);
+  return T <= kG2LowMaxTokens ? launch_gemm2_tiled<true>(T, w2, w2_scale, L, ws, stream)
+                              : launch_gemm2_tiled<false>(T, w2, w2_scale, L, ws, stream);
 }
 
 }  // namespace moe
