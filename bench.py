@@ -58,13 +58,13 @@ def log(*a):
 def stage_work(stage, T, n_sel, a_act):
     """(algorithmic bytes, flops, peak FLOP/s) of one launch of a stage."""
     # bytes: weights and scales once, token rows once, intermediates once each
-    # way (act: bf16 hi + lo = 4 B per value; GEMM2 rows: fp32, or for T <= 64
+    # way (act: bf16 hi + lo = 4 B per value; GEMM2 rows: fp32, or for T <= 8
     # the bf16 output written by GEMM2 itself)
     if stage == "gemm1_swiglu":
         return (a_act * G1_BYTES_PER_EXPERT + T * (H + 56 * 4) + n_sel * I * 4,
                 n_sel * G1_FLOPS_PER_PAIR, PEAK["fp8"])
     if stage == "gemm2":
-        rows_out = T * H * 2 if T <= 64 else n_sel * H * 4
+        rows_out = T * H * 2 if T <= 8 else n_sel * H * 4
         return (a_act * G2_BYTES_PER_EXPERT + n_sel * I * 4 + rows_out,
                 n_sel * G2_FLOPS_PER_PAIR, PEAK["bf16"])
     if stage == "route":

@@ -91,7 +91,7 @@ int moe_fp8_ds_run(const float* routing_logits, const void* routing_bias,
  *
  * The intermediates live in a static device array inside the library, sized
  * for MOE_FP8_DS_NOALLOC_MAX_TOKENS tokens (decode and small batches; the
- * workspace size for 64 tokens, about 4.2 MB, held on every device the library runs on until the process ends).
+ * workspace size for 64 tokens, about 19 MB, held on every device the library runs on until the process ends).
  * T above that returns MOE_FP8_DS_ERR_SCRATCH.  The call allocates nothing
  * and, like moe_fp8_ds_run, needs no initialised scratch.  It uses the
  * scratch of the current device (the stream must belong to it), and every
@@ -107,7 +107,7 @@ int moe_fp8_ds_run_noalloc(const float* routing_logits, const void* routing_bias
 
 /* Number of device stages of moe_fp8_ds_run: routing + permutation, GEMM1 +
  * SwiGLU, GEMM2, combine.  For T <= 16 the routing runs inside GEMM1 (stage 0
- * is empty), and for T <= 64 the combine inside GEMM2 (stage 3 is empty). */
+ * is empty), and for T <= 8 the combine inside GEMM2 (stage 3 is empty). */
 #define MOE_FP8_DS_NUM_STAGES 4
 
 /* moe_fp8_ds_run, plus a hipEventRecord on `stream` before the first stage and
@@ -143,8 +143,8 @@ typedef struct {
                         per 64-column chunk c, 64 hi then 64 lo bf16 (8 KB/row).
                         T >= 1024 with two or more local experts that every token
                         selects: their rows times the routing weight              */
-  size_t down;       /* float [8T, 7168] GEMM2 output rows (T > 64 only; for
-                        T <= 64 GEMM2 combines in registers and the region is empty).
+  size_t down;       /* float [8T, 7168] GEMM2 output rows (T > 8 only; for
+                        T <= 8 GEMM2 combines in LDS and the region is empty).
                         Experts every token selects (as for act): the first one's
                         rows hold each token's weighted sum over all of them, the
                         others' rows are not written                              */

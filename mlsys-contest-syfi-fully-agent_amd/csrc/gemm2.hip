@@ -13,7 +13,7 @@
 // reference CUDA's own hi/lo design; a single bf16 C fails the 1e-2 check on
 // several percent of the elements once outputs reach ~1e3.
 //
-// Two kernels: a streaming one for T <= 64 (weights read once, the
+// Two kernels: a streaming one for T <= 8 (weights read once, the
 // routing-weighted combine fused in) and an LDS-tiled one for larger T (fp32
 // rows to the combine pass), with tiles of their own for experts of few rows.
 #include <type_traits>
@@ -27,12 +27,12 @@ namespace {
 // Streaming path with the combine fused in (T <= kGemm2StreamMaxTokens).
 //
 //   * a workgroup owns 32 output columns n0..n0+31 for all T tokens; it walks
-//     the active experts in ascending order (the order of moe.py:168-200) and
-//     their 16-row tiles, computing O = act_rows . W2_e[n0..n0+31]^T
+//     the active experts in ascending order (the order of moe.py:168-200; an
+//     expert has at most T rows), computing O = act_rows . W2_e[n0..n0+31]^T
 //     (two 16-column MFMA blocks: each job's act rows are loaded once for
 //     32 columns, which halves their L2 traffic against 16-column groups);
 //   * its 8 waves split K (2 scale blocks each); the W2 slices of the next
-//     two (expert, row tile) jobs stream into LDS while one is multiplied;
+//     two jobs (experts) stream into LDS while one is multiplied;
 //   * the K-partials are summed in LDS in a fixed order and each row's
 //     O * weight is added to its token's fp32 accumulator in LDS
 //     (acc = acc + O * w, the two roundings of moe.py:199-200); a token occurs
@@ -50,15 +50,10 @@ constexpr int kS2Cols = 16 * kS2NB;       // output columns per workgroup
 constexpr int kS2Units = kH / kS2Cols;    // 224 column groups
 static_assert(kBlk % kS2Cols == 0, "a workgroup's columns share one weight scale block");
 
-struct S2Job {
-  int e, rt;  // expert, row tile; e < 0: none
-};
-
-// Next (expert, row tile) after `j` in ascending expert order (wave-level).
-__device__ __forceinline__ S2Job s2_next(const ExpertRows& X, uint32_t active, S2Job j) {
-  if (j.e >= 0 && (j.rt + 1) * 16 < X.end(j.e) - X.begin(j.e)) return {j.e, j.rt + 1};
-  const uint32_t later = j.e >= 0 ? active & ~((2u << j.e) - 1u) : active;
-  return later ? S2Job{__builtin_ctz(later), 0} : S2Job{-1, 0};
+// Next expert with rows after `e` (-1: the first), or -1.
+__device__ __forceinline__ int s2_next(uint32_t active, int e) {
+  const uint32_t later = e >= 0 ? active & ~((2u << e) - 1u) : active;
+  return later ? __builtin_ctz(later) : -1;
 }
 
 // A job's act operands, 16 slots: slot c = ((k * 2 + g) * 2 + h) * 2 + part
@@ -73,29 +68,27 @@ __device__ __forceinline__ int s2_slot_off(int c) {
 }
 
 struct S2Regs {
-  v4i op[kS2Slots];  // act operands (spread S > 0: over op[0 .. 16 / 2^S), see s2_load)
+  v4i op[kS2Slots / 2];  // act operands (spread S: over op[0 .. 16 / 2^S), see s2_load)
   float sw[kS2KB];
   int tok;           // token and weight of the row this thread combines
-  float pw;          //   (row = (tid / 16) % 16 of the tile)
+  float pw;          //   (row = (tid / 16) % 16 of the job)
 };
 
-// Loads a job's act rows.  The loads cost per instruction, not per lane: a
-// job of one to four rows took 16 of them for 16 rows, on the path its W2
-// copies share (small_t64: 18 of GEMM2's 63 us).  Spread S: every expert of
-// the launch has at most 16 / 2^S rows (so every job), and the 16 slots take
-// 16 / 2^S instructions, lane (q, r) taking row r mod 16 / 2^S of slot
-// 2^S i + r / (16 / 2^S) (S = 2: row r % 4 of slot 4i + r / 4); s2_operand
-// moves them into the MFMA lanes once they have landed.  Chosen per launch,
-// not per job: a branch per job made the compiler merge two layouts of the
-// persistent operand registers and wait for every load in flight before the
-// next job's loads.
+// Loads a job's act rows.  The loads cost per instruction, not per lane, on
+// the path its W2 copies share: spread S (every expert of the launch has at
+// most 16 / 2^S rows) takes the 16 slots in 16 / 2^S instructions, lane (q, r)
+// taking row r mod 16 / 2^S of slot 2^S i + r / (16 / 2^S) (S = 2: row r % 4
+// of slot 4i + r / 4); s2_operand moves them into the MFMA lanes once they
+// have landed.  Chosen per launch, not per job: a branch per job made the
+// compiler merge two layouts of the persistent operand registers and wait for
+// every load in flight before the next job's loads.
 template <int S>
-__device__ __forceinline__ void s2_load(S2Regs& R, S2Job j, const ExpertRows& X,
+__device__ __forceinline__ void s2_load(S2Regs& R, int e, const ExpertRows& X,
                                         const int32_t* __restrict__ perm_token, const float* __restrict__ perm_w,
                                         const uint16_t* __restrict__ act, const float* __restrict__ w2_scale, int n0,
                                         int kb0, int lq, int lr) {
-  const int row0 = X.begin(j.e) + j.rt * 16;
-  const int rows = min(16, X.end(j.e) - row0);
+  const int row0 = X.begin(e);
+  const int rows = X.end(e) - row0;
   // combine operands first: waiting for them never waits for the prefetch
   const int crow = row0 + min((int)(threadIdx.x >> 4) & 15, rows - 1);
   R.tok = perm_token[crow];
@@ -106,7 +99,7 @@ __device__ __forceinline__ void s2_load(S2Regs& R, S2Job j, const ExpertRows& X,
 #pragma unroll
   for (int i = 0; i < kS2Slots >> S; ++i) R.op[i] = *(const v4i*)(ap + s2_slot_off((i << S) + lr / kRows));
 #pragma unroll
-  for (int k = 0; k < kS2KB; ++k) R.sw[k] = w2_scale[((size_t)j.e * kNHBlk + n0 / kBlk) * kNIBlk + kb0 + k];
+  for (int k = 0; k < kS2KB; ++k) R.sw[k] = w2_scale[((size_t)e * kNHBlk + n0 / kBlk) * kNIBlk + kb0 + k];
 }
 
 // v4i of lane r + N of the lane's 16-lane row (DPP row_shl:N; lanes past the
@@ -160,33 +153,19 @@ __device__ __forceinline__ v4i s2_op(const S2Regs& R, int k, int g, int h, int p
 // A job's W2 bytes of this wave (rows n0 .. n0 + 31, K blocks kb0, kb0 + 1)
 // -> the wave's LDS stage: per 16-row block and K block two wide planes (rows
 // 0-7, 8-15), 128 bytes per row, chunks swizzled, so every copy reads 8 whole
-// 128-byte row segments.  8 copies per lane.
-__device__ __forceinline__ void s2_copy_w(char* stage, S2Job j, const ExpertRows& X, const uint8_t* __restrict__ w2,
-                                          int n0, int kb0, int lane) {
-  auto copy = [&](auto nt_c) {
+// 128-byte row segments, once (nt).  8 copies per lane.
+__device__ __forceinline__ void s2_copy_w(char* stage, int e, const uint8_t* __restrict__ w2, int n0, int kb0,
+                                          int lane) {
 #pragma unroll
-    for (int nb = 0; nb < kS2NB; ++nb)
+  for (int nb = 0; nb < kS2NB; ++nb)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        int r, c;
-        wide_copy_lane(lane, h, r, c);
-        const uint8_t* src = w2 + ((size_t)j.e * kH + n0 + 16 * nb + r) * kI + kb0 * kBlk + 16 * c;
+    for (int h = 0; h < 2; ++h) {
+      int r, c;
+      wide_copy_lane(lane, h, r, c);
+      const uint8_t* src = w2 + ((size_t)e * kH + n0 + 16 * nb + r) * kI + kb0 * kBlk + 16 * c;
 #pragma unroll
-        for (int k = 0; k < kS2KB; ++k) {
-          if constexpr (decltype(nt_c)::value)
-            dma16_nt(src + k * kBlk, stage + ((nb * kS2KB + k) * 2 + h) * 1024);
-          else
-            dma16(src + k * kBlk, stage + ((nb * kS2KB + k) * 2 + h) * 1024);
-        }
-      }
-  };
-  // A row tile with more of the expert's row tiles after it: the next job
-  // copies the same W2 slice again, so the lines stay in L2 for it; the
-  // expert's last row tile reads them for the last time.
-  if ((j.rt + 1) * 16 < X.end(j.e) - X.begin(j.e))
-    copy(std::false_type{});
-  else
-    copy(std::true_type{});
+      for (int k = 0; k < kS2KB; ++k) dma16_nt(src + k * kBlk, stage + ((nb * kS2KB + k) * 2 + h) * 1024);
+    }
 }
 
 __global__ void __launch_bounds__(kS2Threads)
@@ -217,9 +196,9 @@ gemm2_combine_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict
   ExpertRows X;
   X.load(expert_off);
   const uint32_t active = X.active();
-  // Jobs in ascending (expert, row tile) order.  The W2 slices of the next
-  // two jobs stream into the wave's two LDS stages while one is multiplied;
-  // the act rows of the next job load into registers.
+  // Jobs: the experts with rows, ascending.  The W2 slices of the next two jobs
+  // stream into the wave's two LDS stages while one is multiplied; the act
+  // rows of the next job load into registers.
   //
   // Act rows are loaded only together with a W2 copy after them (when no job
   // after next exists, a second copy of the job just copied, whose lines are
@@ -228,21 +207,21 @@ gemm2_combine_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict
   // MFMAs counts, along every path, the loads issued after the operands';
   // with a copy that could be skipped alone it merged the paths to vmcnt(0)
   // and so waited for the prefetch it had just issued, one full memory
-  // latency per job (small_t64: 3.6 us per job, 2.1 of it that wait).
-  // Every expert of the launch has at most four rows (every launch at T <= 4,
-  // decode among them) or at most eight: act rows spread over 4 or 8 loads
-  // per job (s2_load), one loop for the whole launch (decode_t1_s3 23.7 ->
-  // 22.6 us, T = 17 84.8 -> 79.0 us, same bits).
-  const int spread = __ballot(X.cnt > 4) == 0 ? 2 : __ballot(X.cnt > 8) == 0 ? 1 : 0;
+  // latency per job.
+  // Every expert of the launch has at most four rows (every launch at T <= 4)
+  // or at most eight: act rows spread over 4 or 8 loads per job (s2_load), one
+  // loop for the whole launch (decode of one token: 23.7 -> 22.6 us).
+  static_assert(kGemm2StreamMaxTokens <= 8, "an expert has at most 8 rows: spread 1 or 2");
+  const bool four = __ballot(X.cnt > 4) == 0;
   auto run = [&](auto spread_c) {
     constexpr int S = decltype(spread_c)::value;
-    S2Job job = s2_next(X, active, {-1, 0});
-    S2Job j1 = job.e >= 0 ? s2_next(X, active, job) : job;
+    int job = s2_next(active, -1);
+    int j1 = job >= 0 ? s2_next(active, job) : job;
     S2Regs r0, r1;
-    if (job.e >= 0) {
+    if (job >= 0) {
       s2_load<S>(r0, job, X, perm_token, perm_w, act, w2_scale, n0, kb0, lq, lr);
-      s2_copy_w(stage(0), job, X, w2, n0, kb0, lane);
-      s2_copy_w(stage(1), j1.e >= 0 ? j1 : job, X, w2, n0, kb0, lane);
+      s2_copy_w(stage(0), job, w2, n0, kb0, lane);
+      s2_copy_w(stage(1), j1 >= 0 ? j1 : job, w2, n0, kb0, lane);
     }
     // One job from stage `s` with act rows `cur`; after its MFMAs, loads the
     // next job's act rows into `nxt` and starts the copy of the job after next
@@ -262,7 +241,7 @@ gemm2_combine_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict
           for (int g = 0; g < 2; ++g)
             b[nb][k][g] = *(const v4i*)(stage(s) + 2 * (nb * kS2KB + k) * 1024 + wide_slot(lr, 4 * g + lq));
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage is read: free for the job after next
-      const S2Job j2 = j1.e >= 0 ? s2_next(X, active, j1) : j1;
+      const int j2 = j1 >= 0 ? s2_next(active, j1) : j1;
   #pragma unroll
       for (int nb = 0; nb < kS2NB; ++nb) {
         v4f acc = {0.f, 0.f, 0.f, 0.f};
@@ -286,18 +265,18 @@ gemm2_combine_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict
       }
       // The next job's loads go out after this job's MFMAs: with the memory
       // queue full their issue stalls, and the MFMAs no longer wait behind it
-      // (small_t64 GEMM2 62.5 -> 61.5 us).
-      if (j1.e >= 0) {
+      // (1 us of 62 at 17 experts).
+      if (j1 >= 0) {
         s2_load<S>(nxt, j1, X, perm_token, perm_w, act, w2_scale, n0, kb0, lq, lr);
-        s2_copy_w(stage(s), j2.e >= 0 ? j2 : j1, X, w2, n0, kb0, lane);
+        s2_copy_w(stage(s), j2 >= 0 ? j2 : j1, w2, n0, kb0, lane);
       }
       lds_barrier();
       {
         // thread = (column block nb, row r, column c): every thread of the workgroup
         static_assert(kS2Threads == kS2NB * 256, "one thread per output of a job");
         const int nb = threadIdx.x >> 8, r = (threadIdx.x >> 4) & 15, c = threadIdx.x & 15;
-        const int row = X.begin(job.e) + job.rt * 16 + r;
-        if (row < X.end(job.e)) {
+        const int row = X.begin(job) + r;
+        if (row < X.end(job)) {
           float o = red[nb * 256 + (threadIdx.x & 255)];
   #pragma unroll
           for (int w = 1; w < kS2Waves; ++w) o += red[(w * kS2NB + nb) * 256 + (threadIdx.x & 255)];
@@ -311,18 +290,16 @@ gemm2_combine_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict
       j1 = j2;
     };
   #pragma unroll 1
-    while (job.e >= 0) {
+    while (job >= 0) {
       step(0, r0, r1);
-      if (job.e < 0) break;
+      if (job < 0) break;
       step(1, r1, r0);
     }
   };
-  if (spread == 2)
+  if (four)
     run(std::integral_constant<int, 2>{});
-  else if (spread == 1)
-    run(std::integral_constant<int, 1>{});
   else
-    run(std::integral_constant<int, 0>{});
+    run(std::integral_constant<int, 1>{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated copy lands before the LDS is released
   for (int i = threadIdx.x; i < T * kS2Cols; i += kS2Threads)
     out[(size_t)(i / kS2Cols) * kH + n0 + (i % kS2Cols)] = f32_to_bf16_rne(outacc[i]);
@@ -345,7 +322,7 @@ gemm2_combine_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict
 //     with scale 1); P accumulates the two stages of a 128-K scale block on
 //     v_mfma_f32_16x16x32_bf16, then acc += P * w_scale[n/128, kb].
 // ---------------------------------------------------------------------------
-// One tile shape serves every T > 64: 64 rows x 256 columns, 8 waves, two
+// One tile shape serves every expert of more than 32 rows: 64 rows x 256 columns, 8 waves, two
 // 32 KB stages, so two workgroups (16 waves) share a CU.  Each stage holds
 // 64 K of the rows' bf16 hi and lo halves (128 + 128 bytes per row) and of
 // 256 W2 rows.  With the activation pair, a three-stage ring (96 KB) would

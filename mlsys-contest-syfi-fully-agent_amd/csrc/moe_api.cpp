@@ -21,7 +21,7 @@ namespace {
 // In host code `scratch` only names the symbol; its device address comes from
 // hipGetSymbolAddress, once per device (noalloc_scratch).
 constexpr size_t kNoAllocScratchBytes = moe::make_layout(MOE_FP8_DS_NOALLOC_MAX_TOKENS).total;
-static_assert(kNoAllocScratchBytes <= (size_t)8 << 20, "the no-allocation scratch stays small");
+static_assert(kNoAllocScratchBytes <= (size_t)24 << 20, "the no-allocation scratch stays small");
 __device__ __align__(256) char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;

@@ -35,8 +35,15 @@ constexpr int64_t kMaxTokens = 1 << 19;
 static_assert(kMaxTokens * kH <= (int64_t)1 << 32, "token row offsets fit in 32 bits");
 
 // Largest T for which GEMM2 also performs the weighted combine: its rows
-// never reach the workspace, and no combine pass runs.
-constexpr int kGemm2StreamMaxTokens = 64;
+// never reach the workspace, and no combine pass runs.  Each of its workgroups
+// loads every expert's act rows (16-row MFMA operands straight from L2, ~4 us
+// a job of more than 8 rows); beyond 8 tokens the tiled kernel's low tiles and
+// a combine pass are faster or tie.  Layer us, fused -> tiled + combine: four
+// hot experts T = 16 99 -> 89, 17 111 -> 93, 51 186 -> 134, 64 202 -> 142, two
+// T = 12 83 -> 76, 8 73.3 -> 72.0, 4 55 -> 58; uniform routing T = 64 157 ->
+// 137, 48 133 -> 124, 33 125 -> 119, 24 113 -> 111, 16 85.3 -> 85.3, 7 64.7 ->
+// 66.8.
+constexpr int kGemm2StreamMaxTokens = 8;
 // From this T on, experts that every token selects are summed inside GEMM2
 // (every_token_experts).  Below it the fused tiles (T / 64 row tiles x 28
 // column tiles, each running several experts' K loops) are too few to fill
@@ -241,7 +248,7 @@ __device__ __forceinline__ void dma16(const void* g, void* lds_wave_base) {
   __builtin_amdgcn_global_load_lds(g, (lds_void*)lds_wave_base, 16, 0, 0);
 }
 // Same with the nontemporal (nt) cache policy, for data read exactly once:
-// the streaming kernels' expert weights (small_t64: GEMM1 101 -> 87 us).  The
+// the streaming kernels' expert weights (T = 64: GEMM1 101 -> 87 us).  The
 // tiled kernels re-read weight tiles through L2 and keep dma16 (nt there made
 // GEMM2 at T = 8192 34% slower).
 __device__ __forceinline__ void dma16_nt(const void* g, void* lds_wave_base) {

@@ -29,7 +29,7 @@ H, I, E_LOCAL, E_GLOBAL, TOP_K, BLOCK = 7168, 2048, 32, 256, 8, 128
 # Up to this T the GEMM2 kernel also performs the weighted combine and the
 # workspace holds no GEMM2 rows (`down`; kGemm2StreamMaxTokens in
 # csrc/moe_common.hpp).
-FUSED_COMBINE_MAX_TOKENS = 64
+FUSED_COMBINE_MAX_TOKENS = 8
 # Up to this T one workgroup routes the tokens and builds the permutation
 # (inside GEMM1 for T <= 16 in the layer), so the workspace holds no
 # per-workgroup routing histograms (`block_hist`; kRouteSingleMaxTokens in

@@ -34,6 +34,10 @@ def tokens_with_rows(pkg, cfg, device, T, counts):
 
 # (T, rows per expert, tokens and rows checked: None = all)
 ROW_CASES = [
+    (9, (9, 1, 8), None),                # smallest T with GEMM2 rows and a combine pass
+    (16, (16, 15, 1, 16, 9), None),
+    (17, (17, 16, 1), None),
+    (64, (64, 33, 32, 17, 16, 1), None),
     (65, (1, 15, 16, 17, 31, 32, 33, 48, 64, 65), None),
     (130, (16, 1, 130, 32, 2, 128, 64, 33), None),
     (700, (32,) * 20 + (16,) * 8 + (31, 17, 8, 1), None),
