@@ -10,8 +10,10 @@
 // Design (gfx950): HBM-bound (reads 2 B and writes 1 B per element), so the
 // arithmetic per element has to stay under the memory time.  Up to T = 2048
 // one workgroup per token row, wave p quantising pass p (7 waves per row, so
-// that enough loads are in flight at small T).  Beyond, one wave per token
-// row, four rows per workgroup (T/4 workgroups: 2048 at T = 8192).  A
+// that enough loads are in flight at small T).  From T = 5120, where the rows
+// outgrow the caches, half a row per wave with nontemporal loads
+// (quantize_hidden_stream_kernel).  Between, one wave per token
+// row, four rows per workgroup (T/4 workgroups: 1024 at T = 4096).  A
 // wave issues all 14 row loads (16 B per lane each) before any arithmetic, so
 // a token has its whole 14 KB row in flight at once; each of the 7 passes
 // then covers 1024 columns = 8 scale blocks, 8 lanes per block and 16
@@ -198,11 +200,77 @@ quantize_hidden_rows_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __re
   if ((lane & (kQLanesPerBlk - 1)) == 0) scale[(size_t)(c * (kQPass / kBlk) + lane / kQLanesPerBlk) * T + t] = s;
 }
 
+// Large T: one wave per half token row, 7 passes of 512 columns.  A lane takes 8
+// elements a pass (16 lanes per scale block), so each load instruction covers
+// 1 KB of contiguous bytes (16 elements per lane would touch every line
+// twice), and the rows, read once, are loaded nontemporally.  Same arithmetic,
+// same bits.  us, one wave per row with temporal loads -> this: T = 14107 58.9
+// -> 54.5, 10000 42.4 -> 37.7 (5.8 TB/s), 8192 35.7 -> 31.6, 5632 25.6 -> 23.5,
+// 5120 22.8 -> 22.1; at T = 4608 a tie, and below it the nontemporal loads lose
+// (4096 17.4 -> 18.4: there the rows are still cached).  Nontemporal stores
+// gained another 0-4 % but would send the layer's input past the caches.
+constexpr int kQStreamMinTokens = 5120;
+constexpr int kQHalf = kH / 2;                     // columns per wave
+constexpr int kQStreamPass = kWave * 8;            // 512 columns
+constexpr int kQStreamPasses = kQHalf / kQStreamPass;  // 7
+static_assert(kQStreamPasses * kQStreamPass == kQHalf && 16 * 8 == kBlk, "whole passes, 16 lanes per scale block");
+
+// One pass of a wave: 8 elements per lane, 16 lanes per scale block.
+__device__ __forceinline__ void quantize_pass8(const v4i& a, uint2& out, float& s) {
+  const uint32_t e[4] = {(uint32_t)a[0], (uint32_t)a[1], (uint32_t)a[2], (uint32_t)a[3]};
+  uint32_t m = 0, ok = 0;  // largest magnitude (bf16 bits), with and without NaN elements
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m = max(m, max(e[i] & 0x7FFFu, (e[i] >> 16) & 0x7FFFu));
+  m = row16_max_u32(m);
+  const bool odd = m > 0x7F7Fu || (m != 0u && m < kQTinyBf16);
+  if (__ballot(odd) == 0) {
+    const float amax = __uint_as_float(m << 16);
+    s = amax > 0.0f ? amax / 448.0f : 1.0f;
+    const float r = 1.0f / s;
+    out.x = fast_pack4(bf16_lo(e[0]), bf16_hi(e[0]), bf16_lo(e[1]), bf16_hi(e[1]), s, r);
+    out.y = fast_pack4(bf16_lo(e[2]), bf16_hi(e[2]), bf16_lo(e[3]), bf16_hi(e[3]), s, r);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t lo = e[i] & 0x7FFFu, hi = (e[i] >> 16) & 0x7FFFu;
+      ok = max(ok, max(lo > 0x7F80u ? 0u : lo, hi > 0x7F80u ? 0u : hi));
+    }
+    const float amax = __uint_as_float(row16_max_u32(ok) << 16);
+    s = amax > 0.0f ? amax / 448.0f : 1.0f;
+    out.x = exact_pack4(bf16_lo(e[0]), bf16_hi(e[0]), bf16_lo(e[1]), bf16_hi(e[1]), s);
+    out.y = exact_pack4(bf16_lo(e[2]), bf16_hi(e[2]), bf16_lo(e[3]), bf16_hi(e[3]), s);
+  }
+}
+
+__global__ void __launch_bounds__(kWave)
+quantize_hidden_stream_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __restrict__ q,
+                              float* __restrict__ scale) {
+  const int t = blockIdx.x >> 1, c0 = (blockIdx.x & 1) * kQHalf;
+  const int lane = threadIdx.x;
+  const uint16_t* src = x + (size_t)t * kH + c0 + lane * 8;
+  uint8_t* dst = q + (size_t)t * kH + c0 + lane * 8;
+  v4i raw[kQStreamPasses];
+#pragma unroll
+  for (int c = 0; c < kQStreamPasses; ++c) raw[c] = __builtin_nontemporal_load((const v4i*)(src + c * kQStreamPass));
+#pragma unroll
+  for (int c = 0; c < kQStreamPasses; ++c) {
+    uint2 out;
+    float s;
+    quantize_pass8(raw[c], out, s);
+    *(uint2*)(dst + c * kQStreamPass) = out;
+    if ((lane & 15) == 0) scale[(size_t)((c0 + c * kQStreamPass) / kBlk + (lane >> 4)) * T + t] = s;
+  }
+}
+
 }  // namespace
 
 hipError_t launch_quantize_hidden(const uint16_t* x, int T, uint8_t* q, float* scale, hipStream_t stream) {
   if (T <= kQSmallMaxTokens) {
     hipLaunchKernelGGL(quantize_hidden_rows_kernel, dim3(T), dim3(kQPasses * kWave), 0, stream, x, T, q, scale);
+    return hipGetLastError();
+  }
+  if (T >= kQStreamMinTokens) {
+    hipLaunchKernelGGL(quantize_hidden_stream_kernel, dim3(2 * T), dim3(kWave), 0, stream, x, T, q, scale);
     return hipGetLastError();
   }
   const int blocks = (T + kQTokens - 1) / kQTokens;

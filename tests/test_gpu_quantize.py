@@ -113,3 +113,20 @@ def test_quantize_fast_and_exact_paths(pkg, orc, cuda_device):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(q.view(torch.uint8).cpu().numpy(), q_ref)
     np.testing.assert_array_equal(sc.cpu().numpy().view(np.uint32), sc_ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("T", [5119, 5120, 5121, 7003])  # half a row per wave from 5120
+def test_quantize_large_t_matches_oracle(pkg, orc, cuda_device, T):
+    """Special rows first, in the middle and last, both halves of a row."""
+    host = _rows(T, seed=T)
+    special = _special_rows()
+    for at in (0, T // 2, T - 3):
+        host[at:at + 3] = special
+        host[at:at + 3, H // 2:] = special[:, :H // 2]
+    q_ref, sc_ref = orc.quantize_hidden(host)
+    x = torch.from_numpy(host.view(np.int16)).view(torch.bfloat16).to(cuda_device)
+    print(f"quantize T={T}", flush=True)
+    q, sc = pkg.quantize_hidden(x)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(q.view(torch.uint8).cpu().numpy(), q_ref)
+    np.testing.assert_array_equal(sc.cpu().numpy().view(np.uint32), sc_ref.view(np.uint32))
