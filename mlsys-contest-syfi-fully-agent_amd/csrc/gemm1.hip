@@ -59,7 +59,7 @@ constexpr int kS1Groups = kI / 8;         // 256 column groups per expert
 constexpr int kS1CopySplit = 4;           // weight copy parts: K blocks [0, 4) and [4, 7)
 constexpr int kS1CopyOps0 = 2 * kS1CopySplit;            // copies per lane, part 0
 constexpr int kS1CopyOps1 = 2 * (kS1KB - kS1CopySplit);  // copies per lane, part 1
-constexpr int kS1TiledLdsBytes = 81280;  // G1TiledPaths<4, 2>::kLdsBytes (checked where it is defined)
+constexpr int kS1TiledLdsBytes = 80768;  // G1TiledPaths<4, 2>::kLdsBytes (checked where it is defined)
 
 // Operands of one 16-row tile that go out before it is multiplied.
 struct S1TileOps {
@@ -95,8 +95,7 @@ __device__ __forceinline__ void gemm1_tiled_run(char* lds, const uint8_t* __rest
                                                 const float* __restrict__ hs_scale, int T,
                                                 const uint8_t* __restrict__ w13, const float* __restrict__ w13_scale,
                                                 const int32_t* __restrict__ expert_off,
-                                                const int32_t* __restrict__ perm_token, const float* __restrict__ perm_w,
-                                                uint16_t* __restrict__ act);
+                                                const int32_t* __restrict__ perm_token, uint16_t* __restrict__ act);
 
 template <bool kDirect>
 __global__ void __launch_bounds__(kS1Threads)
@@ -136,7 +135,7 @@ gemm1_stream_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs
     // tile and the streaming loop would reload them per item; run the tiled
     // kernel's tiles instead (in this kernel's LDS, one workgroup per CU).
     if (__ballot(X.cnt > 16) != 0 && gridDim.x % 8 == 0) {
-      gemm1_tiled_run<4, 2>(lds, hs, hs_scale, T, w13, w13_scale, expert_off, perm_token, nullptr, act);
+      gemm1_tiled_run<4, 2>(lds, hs, hs_scale, T, w13, w13_scale, expert_off, perm_token, act);
       return;
     }
   }
@@ -404,28 +403,16 @@ gemm1_stream_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs
 //   * per K block: P = A_f8 * B_f8 (v_mfma_f32_16x16x128_f8f6f4, exact
 //     products), acc += P * (a_scale[row] * w_scale[n/128]).
 // ---------------------------------------------------------------------------
-// Kernel choice by T: the tiled kernel up to kGemm1TiledLargeMinTokens - 1,
-// both launched up to kGemm1BothMaxTokens (each exits unless the row counts
-// choose it, wide_tiles_full), the wide 256 x 256 tiles beyond.  Both give
-// the same output bits.  The wide tiles pay when a few experts hold most rows
-// (their 256-row tiles then mostly full); with rows spread over many experts
-// the tiled kernel's 64- and 128-row tiles copy less and fill two workgroups
-// per CU.  Interleaved A/B, GEMM1 us, wide -> tiled: prefill routing
-// T = 1025 184.0 -> 139.5, 1280 188.9 -> 146.6, 1536 179.4 -> 167.3, 2048
-// 198.8 -> 198.1; small_t64 routing T = 1100 182.8 -> 147.0, 1536 188.3 ->
-// 166.8, 2048 193.5 -> 191.5; four hot experts T = 1025 196.7 -> 216.6, 1536
-// 268.1 -> 297.2, 2048 317.7 -> 369.0 (wide tile fill 0.20-0.39 without hot
-// experts, 0.54-0.74 with them).  Past T = 1536 the spread case is a tie,
-// and launching both would cost the exiting kernel's ~3 us.
-constexpr int kGemm1TiledLargeMinTokens = 1025;
-constexpr int kGemm1BothMaxTokens = 1536;
-
-// True when the wide kernel's 256-row tiles would be at least 45 % full.
-// Wave-level; the same in every workgroup of both kernels.
-__device__ __forceinline__ bool wide_tiles_full(const ExpertRows& X) {
-  const int rows = __builtin_amdgcn_readlane(lane_scan_incl(X.cnt), kWave - 1);
-  return 100 * rows >= 45 * 256 * X.count_tiles(256);
-}
+// Kernel choice by T: the tiled kernel below kGemm1WideMinTokens, the wide tiles
+// from it on.  Both give the same output bits.  Below it most experts hold few
+// rows and 16 column tiles of each leave the 256 one-workgroup CUs unevenly
+// filled (20 experts: 1.25 rounds), where the tiled kernel's 32 on 512 slots do
+// not.  Interleaved A/B, GEMM1 us, tiled -> wide: prefill routing T = 200 101 ->
+// 117, 512 106 -> 118, 700 121 -> 133, 900 131 -> 135, 1024 152 -> 138, 1280
+// 152 -> 137, 1500 170 -> 149; four hot experts T = 1024 230 -> 217 (and 512
+// 177 -> 139, but T alone does not tell them from the others).
+constexpr int kGemm1WideMinTokens = 1024;
+static_assert(kGemm1WideMinTokens <= kEveryTokenFuseMinTokens, "only the wide kernel folds routing weights in");
 
 template <int WM, int WN, int MI, int ST>
 struct G1Tiled {
@@ -481,8 +468,7 @@ struct G1TiledPaths {
   static constexpr int kThreads = Short::kThreads;
   static constexpr int kGroupM = 4;             // at most this many row tiles (of one expert) per L2 group
   static constexpr int kRingBytes = Short::kRingBytes > Tall::kRingBytes ? Short::kRingBytes : Tall::kRingBytes;
-  static constexpr int kRowWBytes = Tall::BM * 4;  // the tile's routing weights (every_token_experts)
-  static constexpr int kLdsBytes = kRingBytes + Short::kWscBytes + kRowWBytes;
+  static constexpr int kLdsBytes = kRingBytes + Short::kWscBytes;
   static_assert(WM != 4 || WN != 2 || kLdsBytes <= kS1TiledLdsBytes, "the streaming kernel's LDS check");
   // Tall tiles (and the tall-first map) or short tiles only, for a grid of
   // `slots` resident workgroups.  In short-tile units a tall tile costs 1.5,
@@ -519,8 +505,7 @@ __device__ __forceinline__ void gemm1_tile(char* lds, float* wsc, const uint8_t*
                                            const float* __restrict__ hs_scale, int T,
                                            const uint8_t* __restrict__ w13, const float* __restrict__ w13_scale,
                                            const int32_t* __restrict__ perm_token, uint16_t* __restrict__ act,
-                                           int e, int row0, int rows, int j0, bool w_once,
-                                           const float* __restrict__ perm_w, bool fold_w) {
+                                           int e, int row0, int rows, int j0, bool w_once) {
   constexpr int WN = C::kWN, MI = C::kMI;
   // The thread index is opaque to the optimiser: values derived from it are
   // computed per tile, not hoisted out of the tile loop and kept live
@@ -536,7 +521,7 @@ __device__ __forceinline__ void gemm1_tile(char* lds, float* wsc, const uint8_t*
 
   // ---- DMA planes of this wave: planes wave + 8k; the first kAPlanes are
   // hidden rows (A), the rest W13 rows (B).  Sources are a wave-uniform base
-  // plus a 32-bit lane offset, one VGPR per plane (T <= 1024 here, so every
+  // plus a 32-bit lane offset, one VGPR per plane (T < 1024 here, so every
   // offset fits).
   constexpr int kAPlanes = 2 * C::kAFrags / C::kWaves;
   static_assert((2 * C::kAFrags) % C::kWaves == 0, "A planes split evenly over the waves");
@@ -591,10 +576,6 @@ __device__ __forceinline__ void gemm1_tile(char* lds, float* wsc, const uint8_t*
     const int blk = (up ? kI : 0) + j0 + 32 * w_n;
     wsc[i] = w13_scale[((size_t)e * kN2IBlk + blk / kBlk) * kNHBlk + kb];
   }
-  // the rows' routing weights, for the epilogue (every_token_experts)
-  float* roww = wsc + WN * 2 * kNHBlk;
-  if (fold_w)
-    for (int i = tid; i < rows; i += C::kThreads) roww[i] = perm_w[row0 + i];
 
   v4f acc[MI][4];
 #pragma unroll
@@ -677,10 +658,8 @@ __device__ __forceinline__ void gemm1_tile(char* lds, float* wsc, const uint8_t*
         const int r = (wm * MI + mi) * 16 + 4 * lq + i;
         if (r < rows) {
           const float x1 = acc[mi][nj][i], x2 = acc[mi][nj + 2][i];
-          float v = silu_mul(x2, x1);
-          if (fold_w) v = v * roww[r];  // every_token_experts: the routing weight
           uint16_t hi, lo;
-          split_bf16(v, hi, lo);
+          split_bf16(silu_mul(x2, x1), hi, lo);
           uint16_t* p = act + (size_t)(row0 + r) * kActRowElems + act_col(j0 + 32 * wn + 16 * nj + lr);
           p[0] = hi;
           p[64] = lo;
@@ -696,8 +675,7 @@ __device__ __forceinline__ void gemm1_tiled_run(char* lds, const uint8_t* __rest
                                                 const float* __restrict__ hs_scale, int T,
                                                 const uint8_t* __restrict__ w13, const float* __restrict__ w13_scale,
                                                 const int32_t* __restrict__ expert_off,
-                                                const int32_t* __restrict__ perm_token, const float* __restrict__ perm_w,
-                                                uint16_t* __restrict__ act) {
+                                                const int32_t* __restrict__ perm_token, uint16_t* __restrict__ act) {
   using P = G1TiledPaths<WM, WN>;
   float* wsc = (float*)(lds + P::kRingBytes);  // [WN][2][56]
 
@@ -734,42 +712,33 @@ __device__ __forceinline__ void gemm1_tiled_run(char* lds, const uint8_t* __rest
     if (it > 0) block_barrier();  // every wave is done with the previous tile's LDS
     const int j0 = nt * P::Short::kGateCols;
     const bool w_once = X.end(e) - X.begin(e) <= (tall_map ? P::BM : P::Short::BM);  // one row tile
-    const bool fold_w = (every_token_experts(X, T) >> e) & 1u;
     if (rows > P::Short::BM)  // workgroup-uniform
       gemm1_tile<typename P::Tall>(lds, wsc, hs, hs_scale, T, w13, w13_scale, perm_token, act, e, row0, rows, j0,
-                                   w_once, perm_w, fold_w);
+                                   w_once);
     else
       gemm1_tile<typename P::Short>(lds, wsc, hs, hs_scale, T, w13, w13_scale, perm_token, act, e, row0, rows, j0,
-                                    w_once, perm_w, fold_w);
+                                    w_once);
   }
 }
 
 
-// both: launched together with the wide kernel; runs only if the row counts
-// choose the tiled tiles (!wide_tiles_full).
 template <int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN, 4)
 gemm1_tiled_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale, int T,
                    const uint8_t* __restrict__ w13, const float* __restrict__ w13_scale,
                    const int32_t* __restrict__ expert_off, const int32_t* __restrict__ perm_token,
-                   const float* __restrict__ perm_w, uint16_t* __restrict__ act, int both) {
+                   uint16_t* __restrict__ act) {
   using P = G1TiledPaths<WM, WN>;
   // One LDS object: the stage ring, then the weight scale table.  (A second
   // __shared__ array makes the compiler wait for every outstanding LDS DMA
   // before any LDS read, which would serialise the pipeline.)
   __shared__ __attribute__((aligned(1024))) char lds[P::kLdsBytes];
-  float* wsc = (float*)(lds + P::kRingBytes);  // [WN][2][56]
-  {
-    ExpertRows X;
-    X.load(expert_off);
-    if (both && wide_tiles_full(X)) return;  // the wide kernel takes this launch
-  }
-  gemm1_tiled_run<WM, WN>(lds, hs, hs_scale, T, w13, w13_scale, expert_off, perm_token, perm_w, act);
+  gemm1_tiled_run<WM, WN>(lds, hs, hs_scale, T, w13, w13_scale, expert_off, perm_token, act);
 }
 
 template <int WM, int WN>
 hipError_t launch_gemm1_tiled(const uint8_t* hs, const float* hs_scale, int T, const uint8_t* w13,
-                              const float* w13_scale, const Layout& L, char* ws, hipStream_t stream, int both) {
+                              const float* w13_scale, const Layout& L, char* ws, hipStream_t stream) {
   using P = G1TiledPaths<WM, WN>;
   const int64_t pairs = (int64_t)T * kTopK;
   const int64_t mtiles = (pairs + P::Short::BM - 1) / P::Short::BM + (pairs < kELocal ? pairs : kELocal);
@@ -780,84 +749,80 @@ hipError_t launch_gemm1_tiled(const uint8_t* hs, const float* hs_scale, int T, c
   const int64_t blocks = upper < cap ? upper : cap;
   hipLaunchKernelGGL((gemm1_tiled_kernel<WM, WN>), dim3((unsigned)blocks), dim3(P::kThreads), 0,
                      stream, hs, hs_scale, T, w13, w13_scale, (const int32_t*)(ws + L.expert_off),
-                     (const int32_t*)(ws + L.perm_token), (const float*)(ws + L.perm_w), (uint16_t*)(ws + L.act),
-                     both);
+                     (const int32_t*)(ws + L.perm_token), (uint16_t*)(ws + L.act));
   return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// Wide path (large T): 256 rows x 256 MFMA columns per workgroup.
-//
-// A 256 x 256 tile moves (256 + 256) x 128 B per K block for 2 x 256 x 256 x
-// 128 FLOP, a third less per FLOP than 256 x 128 tiles, which were slower.
-// What bounds it is the stage itself (barrier, operand reads, copy issue):
-// with every operand L2-resident (a timing-only copy) it ran only 2 % faster.
-//
-//   * 8 waves as 4 (rows) x 2 (columns); wave tile = 64 rows x (64 gate + the
-//     64 matching up columns), 4 x 8 MFMA blocks, 128 accumulator VGPRs;
+// Wide path (T >= kGemm1WideMinTokens): 256 MFMA columns (128 gate + 128 up)
+// per workgroup, one workgroup of 8 waves per CU, in two heights:
+//   * tall, 256 rows: 8 waves as 4 (rows) x 2 (columns), wave tile 64 rows x
+//     (64 gate + the 64 matching up columns), 4 x 8 MFMA blocks, 128
+//     accumulator VGPRs; two LDS stages of 66 KB.  It moves (256 + 256) x 128 B
+//     per K block for 2 x 256 x 256 x 128 FLOP, a third less per FLOP than 256 x
+//     128 tiles, which were slower.  What bounds it at T = 8192 is power: there
+//     the chip holds 1.88 GHz and a copy of the kernel with the MFMAs alone takes
+//     2,800 cycles a stage (2,280 at T = 4096, 2.33 GHz; 3,180 in all);
+//   * short, up to 128 rows (an expert's last rows, or all of them): waves as 2
+//     x 4, wave tile 64 rows x (32 + 32) columns, three LDS stages of 50 KB.
+//     Such tiles wait for their W13 stream: as half-empty tall tiles, with one
+//     stage in flight, they took nearly as long as full ones.  Two stages in
+//     flight, and all tall tiles before all short ones, took GEMM1 from 272 to
+//     236 us at T = 4096 (prefill routing), 217 to 187 at T = 3000, 195 to 174 at
+//     T = 2000, 574 to 539 at T = 14107; hot experts T = 1451 294 -> 275, 8192
+//     1,094 -> 1,077 (same bits).  64-row tiles on top gained nothing.
+// Common to both:
 //   * the workgroup's 128 gate columns (and its 128 up columns) are one
 //     128-column weight scale block, so one gate and one up scale per K block;
-//   * two LDS stages of 66 KB: the copy of K block kb + 1 runs while K block
-//     kb is multiplied, its DMAs issued between the first MFMAs;
+//   * the copy of a later K block runs while K block kb is multiplied, its DMAs
+//     issued between the first MFMAs;
 //   * the DMA sources are a wave-uniform base plus a 32-bit lane offset
 //     (saddr form), one VGPR per copied plane.
 // ---------------------------------------------------------------------------
+template <int WM_, int WN_, int ST>
 struct G1Wide {
   static constexpr int kWaves = 8;
   static constexpr int kThreads = kWave * kWaves;
-  static constexpr int WM = 4, WN = 2;
+  static constexpr int WM = WM_, WN = WN_;
+  static_assert(WM * WN == kWaves, "8 waves");
   static constexpr int MI = 4;                   // 16-row blocks per wave
-  static constexpr int NJ = 4;                   // 16-column gate blocks per wave (and as many up)
-  static constexpr int BM = 16 * MI * WM;        // 256 rows
+  static constexpr int NJ = 8 / WN;              // 16-column gate blocks per wave (and as many up)
+  static constexpr int BM = 16 * MI * WM;        // rows
   static constexpr int kGateCols = 16 * NJ * WN; // 128 act columns
   static constexpr int kNT = kI / kGateCols;     // 16 column tiles
-  static constexpr int kAFrags = BM / 16;        // 16
+  static constexpr int kAFrags = BM / 16;
   static constexpr int kBFrags = 2 * kGateCols / 16;  // 16: 8 gate + 8 up
   static constexpr int kFrag = 2048;
   static constexpr int kBOff = kAFrags * kFrag;
   static constexpr int kSOff = kBOff + kBFrags * kFrag;
   static constexpr int kStageBytes = kSOff + kWaves * kWave * 4;  // + one 64-dword scale slot per wave
-  static constexpr int kStages = 2;
+  static constexpr int kStages = ST;
   static constexpr int kWscBytes = 2 * kNHBlk * 4;
+  static constexpr int kLdsBytes = kStages * kStageBytes + kWscBytes;
   static constexpr int kPlanes = 2 * (kAFrags + kBFrags);
-  static constexpr int kPlanesPerWave = kPlanes / kWaves;       // 8: 4 A + 4 B
-  static constexpr int kScaleRowsPerWave = BM / kWaves;         // 32
+  static constexpr int kPlanesPerWave = kPlanes / kWaves;
+  static constexpr int kAK = 2 * kAFrags / kWaves;              // of them A planes
+  static constexpr int kScaleRowsPerWave = BM / kWaves;
   static constexpr int kGroupM = 4;
   static_assert(kGateCols == kBlk, "one weight scale block per tile");
   static_assert(kPlanes % kWaves == 0 && (kAFrags * 2) % kWaves == 0, "planes split evenly");
+  static_assert(kPlanesPerWave <= 4 * NJ, "copies behind the column blocks");
   static_assert(kScaleRowsPerWave % 4 == 0 && kScaleRowsPerWave <= kWave, "scale rows per wave");
-  static_assert(kStages * kStageBytes + kWscBytes <= 160 * 1024, "LDS");
+  static_assert(kLdsBytes <= 160 * 1024, "LDS");
 };
+using G1WideTall = G1Wide<4, 2, 2>;   // 256 rows
+using G1WideShort = G1Wide<2, 4, 3>;  // 128 rows
+static_assert(G1WideTall::BM == 2 * G1WideShort::BM && G1WideTall::kNT == G1WideShort::kNT, "tall_first map");
 
-// both: launched together with the tiled kernel; runs only if the row counts
-// choose the wide tiles (wide_tiles_full).
-__global__ void __launch_bounds__(G1Wide::kThreads)
-gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale, int T,
-                  const uint8_t* __restrict__ w13, const float* __restrict__ w13_scale,
-                  const int32_t* __restrict__ expert_off, const int32_t* __restrict__ perm_token,
-                  const float* __restrict__ perm_w, uint16_t* __restrict__ act, int both) {
-  using C = G1Wide;
-  __shared__ __attribute__((aligned(1024))) char lds[C::kStages * C::kStageBytes + C::kWscBytes];
-
-  ExpertRows X;
-  X.load(expert_off);
-  if (both && !wide_tiles_full(X)) return;  // the tiled kernel takes this launch
-  const uint32_t fused = every_token_experts(X, T);
-  // An eighth of every expert's tiles per XCD (xcd_expert_tile): block b
-  // takes tiles b / 8, b / 8 + cap, ... of XCD b % 8, cap being the blocks per
-  // XCD.  The grid has a block per possible tile, so a block nearly always
-  // takes one tile; the loop covers an XCD that holds more than cap (an XCD
-  // holds up to 32 tiles more than an eighth of all).
-  const int xcd = blockIdx.x % 8, cap = gridDim.x / 8;
-#pragma unroll 1
-  for (int li = blockIdx.x / 8;; li += cap) {
-  int mt, nt;
-  if (!xcd_expert_tile(X, xcd, li, C::BM, C::kNT, C::kGroupM, mt, nt)) break;
-  if (li >= cap) block_barrier();  // every wave is done with the previous tile's LDS
-  int e, row0, rows;
-  X.find_tile(mt, C::BM, e, row0, rows);
-  const int j0 = nt * C::kGateCols;
-
+// One tile: `rows` rows of expert e from permuted row row0, act columns j0 ..
+// j0 + 127.  Every wave calls it; the caller's barrier separates consecutive tiles.
+template <class C, bool NT>
+__device__ __forceinline__ void gemm1_wide_tile(char* lds, const uint8_t* __restrict__ hs,
+                                                const float* __restrict__ hs_scale, int T,
+                                                const uint8_t* __restrict__ w13, const float* __restrict__ w13_scale,
+                                                const int32_t* __restrict__ perm_token, uint16_t* __restrict__ act,
+                                                int e, int row0, int rows, int j0, const float* __restrict__ perm_w,
+                                                bool fold_w) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int lane = threadIdx.x & (kWave - 1);
   const int lq = lane >> 4;
@@ -876,7 +841,7 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
     const int frag = plane >> 1, half = plane & 1;
     int fr, chunk;
     wide_copy_lane(lane, half, fr, chunk);
-    if (frag < C::kAFrags) {
+    if (k < C::kAK) {
       const int r = min(frag * 16 + fr, rows - 1);
       off[k] = (uint32_t)perm_token[row0 + r] * kH + 16 * chunk;
       dst[k] = frag * C::kFrag + half * 1024;
@@ -893,24 +858,23 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
       (uint32_t)perm_token[row0 + min(wave * C::kScaleRowsPerWave + (lane < C::kScaleRowsPerWave ? lane : 0), rows - 1)];
   const int sdst = C::kSOff + wave * kWave * 4;
 
-  auto issue_plane = [&](int kb, int k, auto nt_c) {
-    char* base = lds + (kb & 1) * C::kStageBytes;
-    const bool a_plane = k < C::kPlanesPerWave / 2;
-    if (a_plane) {
+  auto issue_plane = [&](int kb, int k) {
+    char* base = lds + kb % C::kStages * C::kStageBytes;
+    if (k < C::kAK) {
       // A fragments wholly past the tile's rows are never read: no copy
       if (((wave + k * C::kWaves) >> 1) * 16 < rows) dma16(hs + kb * kBlk + off[k], base + dst[k]);
-    } else if constexpr (decltype(nt_c)::value) {
+    } else if constexpr (NT) {
       dma16_nt(w13e + kb * kBlk + off[k], base + dst[k]);
     } else {
       dma16(w13e + kb * kBlk + off[k], base + dst[k]);
     }
   };
   auto issue_scale = [&](int kb) {
-    dma4(hs_scale + (size_t)kb * T + stok, lds + (kb & 1) * C::kStageBytes + sdst);
+    dma4(hs_scale + (size_t)kb * T + stok, lds + kb % C::kStages * C::kStageBytes + sdst);
   };
-  auto issue = [&](int kb, auto nt_c) {
+  auto issue = [&](int kb) {
 #pragma unroll
-    for (int k = 0; k < C::kPlanesPerWave; ++k) issue_plane(kb, k, nt_c);
+    for (int k = 0; k < C::kPlanesPerWave; ++k) issue_plane(kb, k);
     issue_scale(kb);
   };
 
@@ -932,8 +896,8 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
   // issued as one burst after the barrier, they filled the memory pipeline
   // and every wave stalled in the issue before its first MFMA (T = 8192:
   // 1,198 -> 1,103 us; one plane per block needed more registers than fit).
-  auto compute = [&](int kb, int kc, auto nt_c) {
-    const char* sb = lds + (kb & 1) * C::kStageBytes;
+  auto compute = [&](int kb, int kc) {
+    const char* sb = lds + kb % C::kStages * C::kStageBytes;
     auto frag = [&](int off_) {
       const char* f = sb + off_;
       const v4i lo = *(const v4i*)(f + slot_lo), hi = *(const v4i*)(f + slot_hi);
@@ -982,7 +946,7 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
         if (h == 0 && kc >= 0) {
 #pragma unroll
           for (int q = 0; q < 2; ++q)
-            if (2 * nj + q < C::kPlanesPerWave) issue_plane(kc, 2 * nj + q, nt_c);
+            if (2 * nj + q < C::kPlanesPerWave) issue_plane(kc, 2 * nj + q);
         }
         if (h == 1 && nj + 1 < 2 * C::NJ) bn = bfrag(nj + 1);
         if (h == 1 && nj == 0) read_scales();
@@ -1010,32 +974,35 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
   // help with the copies.
   const bool wave_live = C::MI * 16 * wm < rows;
 
-  // Step kb: stage kb has landed (the only copy in flight) and every wave has
-  // finished reading stage kb - 1, so after the barrier that buffer takes the
-  // copy of stage kb + 1 while stage kb is multiplied.
-  auto run = [&](auto nt_c) {
-    issue(0, nt_c);
+  // Step kb: stage kb has landed (with three stages kb + 1 may be in flight)
+  // and every wave has finished reading stage kb - 1, so after the barrier
+  // that buffer takes the next copy while stage kb is multiplied.
+  constexpr int kAhead = C::kStages - 1;
+  int ops = C::kPlanesPerWave - C::kAK + 1;  // this wave's copies of one stage
+#pragma unroll
+  for (int k = 0; k < C::kAK; ++k) ops += ((wave + k * C::kWaves) >> 1) * 16 < rows ? 1 : 0;
+#pragma unroll
+  for (int st = 0; st < kAhead; ++st) issue(st);
 #pragma unroll 1
-    for (int kb = 0; kb < kNHBlk - 1; ++kb) {
+  for (int kb = 0; kb < kNHBlk - kAhead; ++kb) {
+    if constexpr (kAhead == 1)
       wait_vmcnt_lgkm0<0>();
-      block_barrier();
-      if (wave_live)
-        compute(kb, kb + 1, nt_c);
-      else
-        issue(kb + 1, nt_c);
-    }
-    wait_vmcnt_lgkm0<0>();
+    else
+      wait_vmcnt_lgkm0_rt(ops);
     block_barrier();
-    if (wave_live) compute(kNHBlk - 1, -1, nt_c);
-  };
-  // The W13 tile of an expert that fits one row tile is read exactly once:
-  // nontemporal copies, a loop of their own (a branch per copy made the
-  // kernel spill).  T = 1025: GEMM1 206.6 -> 191.8 us, T = 4096 302.8 ->
-  // 291.6 us; T = 8192 unchanged (its hot experts span many row tiles).
-  if (X.end(e) - X.begin(e) <= C::BM)
-    run(std::true_type{});
-  else
-    run(std::false_type{});
+    if (wave_live)
+      compute(kb, kb + kAhead);
+    else
+      issue(kb + kAhead);
+  }
+  if constexpr (kAhead == 2) {
+    wait_vmcnt_lgkm0_rt(ops);
+    block_barrier();
+    if (wave_live) compute(kNHBlk - 2, -1);
+  }
+  wait_vmcnt_lgkm0<0>();
+  block_barrier();
+  if (wave_live) compute(kNHBlk - 1, -1);
 
   // ---- SwiGLU epilogue (moe.py:190-193): act = silu(up) * gate ------------
 #pragma unroll
@@ -1045,13 +1012,13 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
       uint16_t* arow = act + (size_t)(row0 + r) * kActRowElems;
       const int c0 = j0 + 16 * C::NJ * wn + 4 * lq;  // 4 adjacent columns: one 8-byte store per half
       // every_token_experts: the row's routing weight folded in
-      const float wr = (fused >> e) & 1u ? perm_w[row0 + r] : 1.0f;
+      const float wr = fold_w ? perm_w[row0 + r] : 1.0f;
 #pragma unroll
       for (int nj = 0; nj < C::NJ; ++nj) {
         float c[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) c[i] = silu_mul(acc[mi][C::NJ + nj][i], acc[mi][nj][i]);
-        if ((fused >> e) & 1u) {
+        if (fold_w) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) c[i] = c[i] * wr;
         }
@@ -1064,18 +1031,65 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
       }
     }
   }
+}
+
+__global__ void __launch_bounds__(G1WideTall::kThreads)
+gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale, int T,
+                  const uint8_t* __restrict__ w13, const float* __restrict__ w13_scale,
+                  const int32_t* __restrict__ expert_off, const int32_t* __restrict__ perm_token,
+                  const float* __restrict__ perm_w, uint16_t* __restrict__ act) {
+  using C = G1WideTall;
+  constexpr int kLds = C::kLdsBytes > G1WideShort::kLdsBytes ? C::kLdsBytes : G1WideShort::kLdsBytes;
+  __shared__ __attribute__((aligned(1024))) char lds[kLds];
+
+  // An eighth of every expert's tiles per XCD, tall ones first
+  // (xcd_tall_first_tile): block b takes tiles b / 8, b / 8 + cap, ... of XCD b % 8,
+  // cap being the blocks per XCD.  The grid has a block per possible tile, so a
+  // block nearly always takes one tile; the loop covers an XCD that holds more
+  // than cap (an XCD holds up to 32 tiles more than an eighth of all).
+  const int xcd = blockIdx.x % 8, cap = gridDim.x / 8;
+#pragma unroll 1
+  for (int li = blockIdx.x / 8;; li += cap) {
+    ExpertRows X;
+    X.load(expert_off);
+    int mt, nt, e, row0, rows;
+    if (!xcd_tall_first_tile(X, xcd, li, C::BM, C::kNT, C::kGroupM, mt, nt)) break;
+    if (li >= cap) lds_barrier();  // every wave is done with the previous tile's LDS
+    X.find_tile(mt, C::BM, e, row0, rows);
+    const int j0 = nt * C::kGateCols;
+    const bool fold_w = (every_token_experts(X, T) >> e) & 1u;
+    // The W13 tile of an expert that fits one row tile is read exactly once:
+    // nontemporal copies, a loop of their own (a branch per copy made the
+    // kernel spill): T = 4096 302.8 -> 291.6 us; T = 8192 unchanged (its hot
+    // experts span many row tiles).
+    const bool once = X.end(e) - X.begin(e) <= C::BM;
+    auto tile = [&](auto cfg, auto nt_c) {
+      gemm1_wide_tile<decltype(cfg), decltype(nt_c)::value>(lds, hs, hs_scale, T, w13, w13_scale, perm_token, act, e,
+                                                            row0, rows, j0, perm_w, fold_w);
+    };
+    if (rows <= G1WideShort::BM) {
+      if (once)
+        tile(G1WideShort{}, std::true_type{});
+      else
+        tile(G1WideShort{}, std::false_type{});
+    } else {
+      if (once)
+        tile(C{}, std::true_type{});
+      else
+        tile(C{}, std::false_type{});
+    }
   }
 }
 
 hipError_t launch_gemm1_wide(const uint8_t* hs, const float* hs_scale, int T, const uint8_t* w13,
-                             const float* w13_scale, const Layout& L, char* ws, hipStream_t stream, int both) {
-  using C = G1Wide;
+                             const float* w13_scale, const Layout& L, char* ws, hipStream_t stream) {
+  using C = G1WideTall;
   const int64_t pairs = (int64_t)T * kTopK;
   const int64_t mtiles = (pairs + C::BM - 1) / C::BM + (pairs < kELocal ? pairs : kELocal);
   const int64_t blocks = ((mtiles * C::kNT + 7) / 8) * 8;
   hipLaunchKernelGGL(gemm1_wide_kernel, dim3((unsigned)blocks), dim3(C::kThreads), 0, stream, hs, hs_scale, T,
                      w13, w13_scale, (const int32_t*)(ws + L.expert_off), (const int32_t*)(ws + L.perm_token),
-                     (const float*)(ws + L.perm_w), (uint16_t*)(ws + L.act), both);
+                     (const float*)(ws + L.perm_w), (uint16_t*)(ws + L.act));
   return hipGetLastError();
 }
 
@@ -1106,13 +1120,8 @@ hipError_t launch_gemm1(const uint8_t* hs, const float* hs_scale, int T, const u
     }
     return hipGetLastError();
   }
-  if (T < kGemm1TiledLargeMinTokens) return launch_gemm1_tiled<4, 2>(hs, hs_scale, T, w13, w13_scale, L, ws, stream, 0);
-  if (T <= kGemm1BothMaxTokens) {
-    const hipError_t e = launch_gemm1_tiled<4, 2>(hs, hs_scale, T, w13, w13_scale, L, ws, stream, 1);
-    if (e != hipSuccess) return e;
-    return launch_gemm1_wide(hs, hs_scale, T, w13, w13_scale, L, ws, stream, 1);
-  }
-  return launch_gemm1_wide(hs, hs_scale, T, w13, w13_scale, L, ws, stream, 0);
+  return T < kGemm1WideMinTokens ? launch_gemm1_tiled<4, 2>(hs, hs_scale, T, w13, w13_scale, L, ws, stream)
+                                 : launch_gemm1_wide(hs, hs_scale, T, w13, w13_scale, L, ws, stream);
 }
 
 }  // namespace moe

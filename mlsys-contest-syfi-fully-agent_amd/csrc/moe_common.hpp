@@ -526,39 +526,6 @@ __device__ __forceinline__ void grouped_tile(const ExpertRows& X, int t, int bm,
   ntile = r / size;
 }
 
-// Tile map that gives each of the 8 XCDs one eighth of every expert's tiles.
-// Each expert's n_e = nt * (row tiles) tiles are taken in the order of
-// grouped_tile (L2 groups of at most gm row tiles sweeping the nt column
-// tiles); XCD x owns the contiguous slice [x n_e / 8, (x + 1) n_e / 8) of each
-// expert, and its l-th tile is found by walking its slices in expert order.
-// Against contiguous eighths of the whole tile order (xcd_tile), where one
-// XCD could hold nothing but a hot expert's full tiles while another held the
-// short tiles of small experts, every XCD now gets the same mix; a hot
-// expert's L2 groups still stay whole on one XCD.  Wave-level; false past
-// the XCD's last tile.
-__device__ __forceinline__ bool xcd_expert_tile(const ExpertRows& X, int x, int l, int bm, int nt, int gm, int& mt,
-                                                int& ntile) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int rt = (X.cnt + bm - 1) / bm;  // lane e < 32: row tiles of expert e (0 elsewhere)
-  const int n = rt * nt;                  // its tiles
-  const int lo = (int)(((int64_t)x * n) / 8), hi = (int)(((int64_t)(x + 1) * n) / 8);
-  const int size = hi - lo;               // its slice on XCD x
-  const int incl = lane_scan_incl(size);
-  if (l >= __builtin_amdgcn_readlane(incl, kWave - 1)) return false;
-  const int e = __builtin_ctzll(__ballot(incl > l));
-  const int i = __builtin_amdgcn_readlane(lo, e) + l - (__builtin_amdgcn_readlane(incl, e) - __builtin_amdgcn_readlane(size, e));
-  const int rte = __builtin_amdgcn_readlane(rt, e);
-  const int tb = __builtin_amdgcn_readlane(lane_scan_incl(rt) - rt, e);  // row tiles before expert e
-  // expert-local index i -> (row tile, column tile) in grouped_tile's order
-  const int ng = (rte + gm - 1) / gm;
-  const int j = min(i / (gm * nt), ng - 1);
-  const int o = i - j * gm * nt;
-  const int rows_g = min(gm, rte - j * gm);
-  mt = tb + j * gm + o % rows_g;
-  ntile = o / rows_g;
-  return true;
-}
-
 // Row tiles of two heights: an expert's row tiles hold bm rows, its last one
 // fewer; a last row tile of at most bm / 2 rows is "short", every other row
 // tile "tall".  Totals over the experts (wave-level, uniform results).
@@ -570,11 +537,16 @@ __device__ __forceinline__ void tall_short_row_tiles(const ExpertRows& X, int bm
 }
 
 // Tile map for those two heights.  XCD x takes an eighth of every expert's
-// tall tiles and an eighth of its short tiles (as xcd_expert_tile does for one
-// height); its list holds all its tall tiles (expert order, grouped_tile order
-// inside an expert) before its short ones, so that the longer tiles start
-// first.  mt is the row tile in ExpertRows::find_tile(mt, bm) numbering.
-// Wave-level; false past the XCD's last tile.
+// tall tiles and an eighth of its short tiles: each expert's n_e = nt * (row
+// tiles) tiles in the order of grouped_tile (L2 groups of at most gm row tiles
+// sweeping the nt column tiles), XCD x the contiguous slice [x n_e / 8, (x + 1)
+// n_e / 8).  Against contiguous eighths of the whole tile order (xcd_tile),
+// where one XCD could hold nothing but a hot expert's full tiles, every XCD
+// gets the same mix, and a hot expert's L2 groups still stay whole on one XCD.
+// An XCD's list holds all its tall tiles (expert order) before its short ones,
+// so that the longer tiles start first.  mt is the row tile in
+// ExpertRows::find_tile(mt, bm) numbering.  Wave-level; false past the XCD's
+// last tile.
 __device__ __forceinline__ bool xcd_tall_first_tile(const ExpertRows& X, int x, int l, int bm, int nt, int gm,
                                                     int& mt, int& ntile) {
   const int rt = (X.cnt + bm - 1) / bm;
