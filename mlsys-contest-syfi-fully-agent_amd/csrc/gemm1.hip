@@ -815,7 +815,7 @@ using G1WideShort = G1Wide<2, 4, 3>;  // 128 rows
 static_assert(G1WideTall::BM == 2 * G1WideShort::BM && G1WideTall::kNT == G1WideShort::kNT, "tall_first map");
 
 // One tile: `rows` rows of expert e from permuted row row0, act columns j0 ..
-// j0 + 127.  Every wave calls it; the caller's barrier separates consecutive tiles.
+// j0 + 127.  Every wave calls it.
 template <class C, bool NT>
 __device__ __forceinline__ void gemm1_wide_tile(char* lds, const uint8_t* __restrict__ hs,
                                                 const float* __restrict__ hs_scale, int T,
@@ -1043,51 +1043,46 @@ gemm1_wide_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs_s
   __shared__ __attribute__((aligned(1024))) char lds[kLds];
 
   // An eighth of every expert's tiles per XCD, tall ones first
-  // (xcd_tall_first_tile): block b takes tiles b / 8, b / 8 + cap, ... of XCD b % 8,
-  // cap being the blocks per XCD.  The grid has a block per possible tile, so a
-  // block nearly always takes one tile; the loop covers an XCD that holds more
-  // than cap (an XCD holds up to 32 tiles more than an eighth of all).
-  const int xcd = blockIdx.x % 8, cap = gridDim.x / 8;
-#pragma unroll 1
-  for (int li = blockIdx.x / 8;; li += cap) {
-    ExpertRows X;
-    X.load(expert_off);
-    int mt, nt, e, row0, rows;
-    if (!xcd_tall_first_tile(X, xcd, li, C::BM, C::kNT, C::kGroupM, mt, nt)) break;
-    if (li >= cap) lds_barrier();  // every wave is done with the previous tile's LDS
-    X.find_tile(mt, C::BM, e, row0, rows);
-    const int j0 = nt * C::kGateCols;
-    const bool fold_w = (every_token_experts(X, T) >> e) & 1u;
-    // The W13 tile of an expert that fits one row tile is read exactly once:
-    // nontemporal copies, a loop of their own (a branch per copy made the
-    // kernel spill): T = 4096 302.8 -> 291.6 us; T = 8192 unchanged (its hot
-    // experts span many row tiles).
-    const bool once = X.end(e) - X.begin(e) <= C::BM;
-    auto tile = [&](auto cfg, auto nt_c) {
-      gemm1_wide_tile<decltype(cfg), decltype(nt_c)::value>(lds, hs, hs_scale, T, w13, w13_scale, perm_token, act, e,
-                                                            row0, rows, j0, perm_w, fold_w);
-    };
-    if (rows <= G1WideShort::BM) {
-      if (once)
-        tile(G1WideShort{}, std::true_type{});
-      else
-        tile(G1WideShort{}, std::false_type{});
-    } else {
-      if (once)
-        tile(C{}, std::true_type{});
-      else
-        tile(C{}, std::false_type{});
-    }
+  // (xcd_tall_first_tile): block b takes tile b / 8 of XCD b % 8, one tile per
+  // block (see launch_gemm1_wide).
+  static_assert(C::kNT % 8 == 0, "every XCD holds kNT / 8 tiles of each row tile");
+  ExpertRows X;
+  X.load(expert_off);
+  int mt, nt, e, row0, rows;
+  if (!xcd_tall_first_tile(X, blockIdx.x % 8, blockIdx.x / 8, C::BM, C::kNT, C::kGroupM, mt, nt)) return;
+  X.find_tile(mt, C::BM, e, row0, rows);
+  const int j0 = nt * C::kGateCols;
+  const bool fold_w = (every_token_experts(X, T) >> e) & 1u;
+  // The W13 tile of an expert that fits one row tile is read exactly once:
+  // nontemporal copies, a loop of their own (a branch per copy made the
+  // kernel spill): T = 4096 302.8 -> 291.6 us; T = 8192 unchanged (its hot
+  // experts span many row tiles).
+  const bool once = X.end(e) - X.begin(e) <= C::BM;
+  auto tile = [&](auto cfg, auto nt_c) {
+    gemm1_wide_tile<decltype(cfg), decltype(nt_c)::value>(lds, hs, hs_scale, T, w13, w13_scale, perm_token, act, e,
+                                                          row0, rows, j0, perm_w, fold_w);
+  };
+  if (rows <= G1WideShort::BM) {
+    if (once)
+      tile(G1WideShort{}, std::true_type{});
+    else
+      tile(G1WideShort{}, std::false_type{});
+  } else {
+    if (once)
+      tile(C{}, std::true_type{});
+    else
+      tile(C{}, std::false_type{});
   }
 }
 
 hipError_t launch_gemm1_wide(const uint8_t* hs, const float* hs_scale, int T, const uint8_t* w13,
                              const float* w13_scale, const Layout& L, char* ws, hipStream_t stream) {
   using C = G1WideTall;
-  const int64_t pairs = (int64_t)T * kTopK;
-  const int64_t mtiles = (pairs + C::BM - 1) / C::BM + (pairs < kELocal ? pairs : kELocal);
-  const int64_t blocks = ((mtiles * C::kNT + 7) / 8) * 8;
-  hipLaunchKernelGGL(gemm1_wide_kernel, dim3((unsigned)blocks), dim3(C::kThreads), 0, stream, hs, hs_scale, T,
+  // A block for every tile there can be: at most 8T rows over 32 experts make
+  // mtiles row tiles, each of them kNT / 8 tiles of every XCD.
+  static_assert(kGemm1WideMinTokens * kTopK >= kELocal, "every local expert can have rows");
+  const int64_t mtiles = ((int64_t)T * kTopK + C::BM - 1) / C::BM + kELocal;
+  hipLaunchKernelGGL(gemm1_wide_kernel, dim3((unsigned)(mtiles * C::kNT)), dim3(C::kThreads), 0, stream, hs, hs_scale, T,
                      w13, w13_scale, (const int32_t*)(ws + L.expert_off), (const int32_t*)(ws + L.perm_token),
                      (const float*)(ws + L.perm_w), (uint16_t*)(ws + L.act));
   return hipGetLastError();
