@@ -47,7 +47,8 @@ LAYER_CASES = [
     # token counts on either side of each kernel-choice boundary
     ("small_t64", None, 17, None),        # first T past the in-GEMM1 routing
     # the hot experts take every token: experts of exactly 4 rows (act rows
-    # spread over 4 loads per GEMM2 job), of 5 and 8 (8 loads) and of 9 (16)
+    # spread over 4 loads per GEMM2 job), of 5 and 8 (8 loads); of 9, the first
+    # T with GEMM2's low tiles and a combine pass
     ("skewed_t8192", None, 4, None),
     ("skewed_t8192", None, 5, None),
     ("skewed_t8192", None, 8, None),
@@ -59,17 +60,17 @@ LAYER_CASES = [
     ("skewed_t8192", None, 17, None),
     ("skewed_t8192", None, 64, None),
     ("skewed_t8192", None, 40, None),
-    ("prefill_t1024", None, 65, None),    # first T with the tiled GEMM1 and a combine pass
+    ("prefill_t1024", None, 65, None),    # first T with the tiled GEMM1
     # tiled GEMM1 tall tiles: two tall + one short tile of exactly 64 rows per
     # hot expert; prefill routing with tall and short tiles
     ("skewed_t8192", None, 320, None),
     ("prefill_t1024", None, 704, None),
-    ("skewed_t8192", None, 1024, None),   # largest T of the tiled GEMM1 alone
-    # 1025 <= T <= 1536: both GEMM1 kernels launched, the row counts choose one
-    ("skewed_t8192", None, 1025, None),   # four hot experts: the wide kernel runs
-    ("prefill_t1024", None, 1025, None),  # rows spread: the tiled kernel runs
-    ("small_t64", None, 1536, None),      # the same at the range's top
-    ("prefill_t1024", None, 1537, None),  # the wide kernel alone
+    ("skewed_t8192", None, 1023, None),   # largest T of the tiled GEMM1, below the fused experts
+    ("skewed_t8192", None, 1024, None),   # first T of the wide GEMM1, of fused experts
+    ("skewed_t8192", None, 1025, None),   # four hot experts: tall tiles
+    ("prefill_t1024", None, 1025, None),  # rows spread: short tiles
+    ("small_t64", None, 1536, None),
+    ("prefill_t1024", None, 1537, None),
     ("skewed_t8192", None, 2047, None),
     ("skewed_t8192", None, 2048, None),
     ("skewed_t8192", None, 4095, None),
@@ -103,7 +104,7 @@ def test_layer_matches_oracle(pkg, orc, cuda_device, name, offset, T, n_check):
 
 # Other weights and tokens: generator seeds no config uses, each with another
 # local window and a T on another kernel path (streaming, tiled with and
-# without tall tiles, the two-kernel range, wide GEMM1).
+# without tall tiles, wide GEMM1).
 SEED_CASES = [(5, 64, 50), (7, 160, 600), (9, 224, 1500), (11, 0, 800), (13, 96, 1100)]
 
 
@@ -118,8 +119,8 @@ def test_layer_seed_sweep(pkg, orc, cuda_device, seed, offset, T):
     check_layer(pkg, orc, cuda_device, cfg, offset, tok, host, w, w_host, None)
 
 
-# A sweep over the tiled GEMM1's range and the two-kernel range (T = 65 to
-# 1,536 in steps of 122): tile maps with and without tall tiles, every token.
+# A sweep over the tiled GEMM1's range and the first of the wide one's (T = 65
+# to 1,536 in steps of 122): tile maps with and without tall tiles, every token.
 SWEEP_CASES = [(name, T) for name in ("skewed_t8192", "prefill_t1024") for T in range(65, 1537, 122)]
 
 
@@ -159,8 +160,8 @@ def test_layer_other_scaling_factors(pkg, orc, cuda_device, name, rsf, T):
 # holds): +10 on the bias of the 32 local experts puts their group first and
 # all 8 picks in it, for every token, so the experts hold about T / 4 rows
 # each -- experts of more than 16 rows in the streaming kernels at T = 64,
-# tall tiles at T = 300, the two-kernel range (the wide tiles chosen) at
-# T = 1100 and the wide GEMM1 alone at T = 3000.
+# tall tiles at T = 300, the wide GEMM1's tall and short tiles at T = 1100 and
+# 3000.
 ALL_LOCAL_CASES = [(1, None), (16, None), (64, None), (300, None), (1100, 256), (3000, 256)]
 
 
@@ -287,12 +288,12 @@ def test_layer_matches_reference_golden(pkg, cuda_device, name):
 
 
 INTERMEDIATE_CASES = [
-    ("small_t64", None, None),          # row-streaming kernels
+    ("small_t64", None, None),          # row-streaming GEMM1, GEMM2's low tiles
     ("skewed_t8192", 64, None),         # streaming GEMM1 launch with tiled tiles (experts of 64 rows)
     ("prefill_t1024", None, 200),
     ("skewed_t8192", 2304, 160),        # LDS-tiled / wide kernels, ragged last tiles
-    # tiled GEMM2 with experts of a few to ~40 rows, every row: 16-row blocks
-    # past a tile's rows are skipped per wave (0, 1 or 2 live blocks)
+    # GEMM2 with experts of a few to ~60 rows, every row: low tiles up to 32,
+    # full tiles beyond (16-row blocks past a tile's rows skipped per wave)
     ("prefill_t1024", 320, None),
     ("small_t64", 256, None),
     # tiled GEMM1 tile heights (64-row short tiles, 128-row tall tiles, chosen
@@ -303,8 +304,8 @@ INTERMEDIATE_CASES = [
     ("skewed_t8192", 321, 400),         # tall map, three tall tiles, the last of 65 rows
     ("prefill_t1024", 704, 400),        # tall map, partly filled tall tiles among short ones
     # experts of every token summed inside GEMM2 (EVERY_TOKEN_FUSE_MIN_TOKENS):
-    # weights folded in by the tiled GEMM1 (T = 1024) and the wide one (T =
-    # 1100: the hot experts choose it), fused tiles with a ragged last row tile
+    # weights folded in by the wide GEMM1, whole fused tiles (T = 1024) and a
+    # ragged last row tile (T = 1100)
     ("skewed_t8192", 1024, 300),
     ("skewed_t8192", 1100, 300),
 ]
@@ -366,7 +367,7 @@ def test_intermediates_match_oracle(pkg, orc, cuda_device, name, T, n_rows):
     assert not bad_c.any(), f"act: {int(bad_c.sum())} bad, rows {np.unique(np.nonzero(bad_c)[0])[:8]}"
     if T <= pkg.moe.FUSED_COMBINE_MAX_TOKENS:
         assert r.down is None
-        return  # GEMM2 rows are combined in registers, never stored
+        return  # GEMM2 rows are combined in LDS, never stored
     down = r.down[torch.as_tensor(sel, device=r.down.device)].cpu().numpy()
     written = ~in_fused | (le_all[sel] == (fused[0] if fused.size else -1))
     down, o_ref = down[written], o_ref[written]

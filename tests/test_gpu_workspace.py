@@ -89,12 +89,19 @@ def test_captured_workspace_outlives_growth(pkg, cuda_device):
     pkg.release_workspaces()
 
 
-@pytest.mark.parametrize("name,T", [("small_t64", 1100), ("skewed_t8192", 1025)])
-def test_graph_replay_with_both_gemm1_kernels(pkg, cuda_device, name, T):
-    """For 1,025-1,536 tokens the layer launches both GEMM1 kernels and the
-    row counts choose one (the tiled kernel for spread rows, the wide one for
-    hot experts).  A graph of such a call replays to the eager bits, with
-    eager work between the replays."""
+# (routing, T): calls in which the device chooses from the row counts -- GEMM2's
+# low tiles and a combine pass (T = 12), the streaming GEMM1 running tiled
+# tiles (hot experts, T = 40), the tiled GEMM1's short and tall maps and GEMM2's
+# full and low tiles (T = 300, hot experts T = 512), the wide GEMM1's two tile
+# heights (T = 1100), experts of every token summed in GEMM2 (T = 1025)
+DEVICE_CHOICE_CASES = [("prefill_t1024", 12), ("skewed_t8192", 40), ("small_t64", 300), ("skewed_t8192", 512),
+                       ("small_t64", 1100), ("skewed_t8192", 1025)]
+
+
+@pytest.mark.parametrize("name,T", DEVICE_CHOICE_CASES)
+def test_graph_replay_where_the_device_chooses(pkg, cuda_device, name, T):
+    """A graph of such a call replays to the eager bits, with eager work
+    between the replays."""
     cfg = pkg.synth.CONFIGS[name]
     w, _ = gpu_weights(pkg, cfg.seed, cuda_device)
     tok, _ = gpu_tokens(pkg, cfg, cuda_device, T)
