@@ -435,7 +435,7 @@ struct G1Tiled {
   static constexpr int kStageBytes = kSOff + kWaves * kWave * 4;
   static constexpr int kWscBytes = WN * 2 * kNHBlk * 4;  // weight block scales (after the stages)
   static constexpr int kStages = ST;
-  static_assert(kStages >= 2 && kStages <= 6, "pipeline depth (wait_stages_ahead)");
+  static_assert(kStages == 2 || kStages == 3, "pipeline depth (wait_stages_ahead)");
   static constexpr int kRingBytes = kStages * kStageBytes;
   static constexpr int kPlanes = 2 * (kAFrags + kBFrags);
   static_assert(kPlanes % kWaves == 0, "planes must split evenly over waves");

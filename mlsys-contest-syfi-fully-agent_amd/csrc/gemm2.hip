@@ -355,7 +355,6 @@ struct G2Tiled {
   static constexpr int kStageBytes = kBOff + kBFrags * 1024;
   static constexpr int kWscBytes = kTopK * WN * kNIBlk * 4;  // weight block scales of up to 8 experts (after the stages)
   static constexpr int kStages = STAGES;
-  static_assert(kStages >= 2 && kStages <= 5, "pipeline depth");
   static constexpr int kSteps = kI / 64;  // stages per tile (two per scale block)
   static constexpr int kPlanes = kAPlanes + kBFrags;
   static_assert(kPlanes % kWaves == 0, "planes must split evenly over waves");
@@ -405,12 +404,11 @@ struct G2Low {
   static constexpr int kFrag = 2048;             // 16 W2 rows x 128 K
   static constexpr int kWSlot = NF * kFrag;
   static constexpr int kWOps = 2 * NF;           // copies per wave of one K block
-  static constexpr int D = 2;                    // W2 slots per wave
   static constexpr int kAFrag = 4096;            // 16 act rows x 64 K: hi (two wide planes), lo (two)
   static constexpr int KH = RB == 1 ? 2 : 1;     // half steps (64 K) per A stage
   static constexpr int kAStage = RB * KH * kAFrag;
   static_assert(RB * KH * 4 == kWaves, "one A plane per wave and stage");
-  static constexpr int kAOff = kWaves * D * kWSlot;
+  static constexpr int kAOff = kWaves * 2 * kWSlot;  // after two W2 slots per wave
   static constexpr int kLdsBytes = kAOff + 2 * kAStage;
 };
 
@@ -418,7 +416,7 @@ template <class C>
 __device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __restrict__ act,
                                                const uint8_t* __restrict__ w2, const float* __restrict__ w2_scale,
                                                float* __restrict__ down, int e, int row0, int rows, int n0) {
-  constexpr int RB = C::RB, NF = C::NF, D = C::D, KH = C::KH;
+  constexpr int RB = C::RB, NF = C::NF, KH = C::KH;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int lane = threadIdx.x & (kWave - 1);
   const int lq = lane >> 4;
@@ -426,7 +424,7 @@ __device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __rest
   const int nw = n0 + C::kWaveCols * wave;  // the wave's first column
   const char* wbase = (const char*)(w2 + ((size_t)e * kH + nw) * kI);
   const char* abase = (const char*)(act + (size_t)row0 * kActRowElems);
-  char* wring = lds + wave * (D * C::kWSlot);
+  char* wring = lds + wave * (2 * C::kWSlot);
   char* aring = lds + C::kAOff;
   uint32_t woff[2];  // column block 0, rows 0-7 / 8-15
 #pragma unroll
@@ -446,7 +444,7 @@ __device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __rest
   auto issue_w = [&](int kb) {
     uint32_t ko = kb * kBlk;
     asm volatile("" : "+s"(ko));  // added at use: no strength-reduced copies of the offsets
-    char* wslot = wring + (kb % D) * C::kWSlot;
+    char* wslot = wring + (kb & 1) * C::kWSlot;
 #pragma unroll
     for (int c = 0; c < NF; ++c)
 #pragma unroll
@@ -470,7 +468,7 @@ __device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __rest
   v4i raw[NF][2];
   issue_a(0);
   issue_w(0);
-  if (D == 2) issue_w(1);
+  issue_w(1);
   if (RB == 2) issue_a(1);
   // Half step h = 2 kb + g of 64 K; LEFT: K blocks after this one (2: at least
   // two).  Each wait leaves what was issued after the half step's operands:
@@ -480,17 +478,17 @@ __device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __rest
     const int h = 2 * kb + g;
     if constexpr (RB == 1) {
       if (g == 0) {
-        wait_vmcnt_lgkm0<D == 2 && LEFT >= 1 ? C::kWOps : 0>();
+        wait_vmcnt_lgkm0<LEFT >= 1 ? C::kWOps : 0>();
         block_barrier();
         if (LEFT >= 1) issue_a(kb + 1);
       }
     } else {
-      wait_vmcnt_lgkm0<g == 0 ? (D == 2 && LEFT >= 1 ? C::kWOps : 0) + 1
-                              : (LEFT >= D ? C::kWOps : 0) + (LEFT >= 1 ? 1 : 0)>();
+      wait_vmcnt_lgkm0<g == 0 ? (LEFT >= 1 ? C::kWOps : 0) + 1
+                              : (LEFT >= 2 ? C::kWOps : 0) + (LEFT >= 1 ? 1 : 0)>();
       block_barrier();
     }
     if (g == 0) {
-      const char* wslot = wring + (kb % D) * C::kWSlot;
+      const char* wslot = wring + (kb & 1) * C::kWSlot;
 #pragma unroll
       for (int c = 0; c < NF; ++c) {
         raw[c][0] = *(const v4i*)(wslot + c * C::kFrag + slot_b0);
@@ -514,7 +512,7 @@ __device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __rest
     } else if (g == 0) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the W2 slot is read: free for block kb + 2
     }
-    if (g == 0 && LEFT >= D) issue_w(kb + D);
+    if (g == 0 && LEFT >= 2) issue_w(kb + 2);
 #pragma unroll
     for (int c = 0; c < NF; ++c) {
       const v8bf b0 = e4m3x8_to_bf16((uint32_t)raw[c][g][0], (uint32_t)raw[c][g][1]);
@@ -736,8 +734,7 @@ gemm2_tiled_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__
   static_assert(C::kStages == 2, "skipped copies leave the per-stage counts unequal: every wait is for all");
   auto step = [&](int s, bool first, auto live_c) {
     constexpr int L = decltype(live_c)::value;  // live 16-row blocks of this wave
-    // stages s+1 .. s+kStages-2 may stay in flight
-    wait_stages_ahead<C::kPlanesPerWave>(min(n_steps - 1 - s, C::kStages - 2));
+    wait_vmcnt_lgkm0<0>();  // stage s, the only copy in flight
     block_barrier();
     if (s + C::kStages - 1 < n_steps) issue(s + C::kStages - 1);
 

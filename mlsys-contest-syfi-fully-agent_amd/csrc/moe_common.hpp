@@ -199,15 +199,6 @@ __device__ __forceinline__ float float_from_order_key(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int mask) {
-  uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-  lo = __shfl_xor(lo, mask, kWave);
-  hi = __shfl_xor(hi, mask, kWave);
-  return ((uint64_t)hi << 32) | lo;
-}
-
-__device__ __forceinline__ uint64_t u64max(uint64_t a, uint64_t b) { return a > b ? a : b; }
-
 // D = A(16x128 e4m3) * B(128x16 e4m3), fp32 16x16 result (no accumulate-in).
 // Lane l supplies 32 K-bytes of row (l % 16) of A and of column (l % 16) of
 // B; lanes l/16 = 0..3 cover the four 32-byte quarters of the 128 K values.
@@ -247,10 +238,11 @@ typedef __attribute__((address_space(3))) void lds_void;
 __device__ __forceinline__ void dma16(const void* g, void* lds_wave_base) {
   __builtin_amdgcn_global_load_lds(g, (lds_void*)lds_wave_base, 16, 0, 0);
 }
-// Same with the nontemporal (nt) cache policy, for data read exactly once:
-// the streaming kernels' expert weights (T = 64: GEMM1 101 -> 87 us).  The
-// tiled kernels re-read weight tiles through L2 and keep dma16 (nt there made
-// GEMM2 at T = 8192 34% slower).
+// Same with the nontemporal (nt) cache policy, for weights that a launch reads
+// exactly once: the streaming kernels' (T = 64: GEMM1 101 -> 87 us), those of an
+// expert of one row tile in the tiled and wide GEMM1, and GEMM2's low tiles'.
+// Weight tiles that several row tiles read through L2 keep dma16 (nt there
+// made GEMM2 at T = 8192 34% slower).
 __device__ __forceinline__ void dma16_nt(const void* g, void* lds_wave_base) {
   __builtin_amdgcn_global_load_lds(g, (lds_void*)lds_wave_base, 16, 0, 2);
 }
@@ -276,19 +268,11 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-// Waits until at most `ahead` pipeline stages of `per_stage` vector-memory
-// operations each are still in flight (ahead = 0, 1, 2, 3).
+// Waits until at most `ahead` pipeline stages (0 or 1) of `per_stage`
+// vector-memory operations each are still in flight.
 template <int per_stage>
 __device__ __forceinline__ void wait_stages_ahead(int ahead) {
-  if (ahead >= 5)
-    wait_vmcnt_lgkm0<5 * per_stage>();
-  else if (ahead == 4)
-    wait_vmcnt_lgkm0<4 * per_stage>();
-  else if (ahead == 3)
-    wait_vmcnt_lgkm0<3 * per_stage>();
-  else if (ahead == 2)
-    wait_vmcnt_lgkm0<2 * per_stage>();
-  else if (ahead == 1)
+  if (ahead == 1)
     wait_vmcnt_lgkm0<per_stage>();
   else
     wait_vmcnt_lgkm0<0>();
@@ -450,12 +434,6 @@ struct ExpertRows {
   __device__ __forceinline__ int end(int e) const { return __builtin_amdgcn_readlane(o, e + 1); }
   // Bit e set <=> expert e has rows.
   __device__ __forceinline__ uint32_t active() const { return (uint32_t)__ballot(cnt > 0); }
-  // The slot-th expert with rows, or -1.
-  __device__ __forceinline__ int nth_active(int slot) const {
-    uint32_t m = active();
-    for (int k = 0; k < slot && m; ++k) m &= m - 1;
-    return m ? __builtin_ctz(m) : -1;
-  }
   // Inclusive scan over experts of the number of row tiles of height bm.
   __device__ __forceinline__ int tiles_incl(int bm) const { return lane_scan_incl((cnt + bm - 1) / bm); }
   __device__ __forceinline__ int count_tiles(int bm) const {
