@@ -68,34 +68,38 @@ __device__ __forceinline__ uint32_t f32_to_e4m3_satfinite(float x) {
 __device__ __forceinline__ float bf16_lo(uint32_t u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); }
 
-// Largest bf16 magnitude (as bits, 0..0x7FFF) of the 16 elements of one lane;
-// NaN patterns (> 0x7F80) order above every number, so a NaN shows as > 0x7F80.
-__device__ __forceinline__ uint32_t lane_absmax_bits(const uint4& a, const uint4& b) {
-  const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+// Largest bf16 magnitude (as bits, 0..0x7FFF) of one lane's 2N elements; NaN
+// patterns (> 0x7F80) order above every number, so a NaN shows as > 0x7F80.
+template <int N>
+__device__ __forceinline__ uint32_t lane_absmax_bits(const uint32_t (&e)[N]) {
   uint32_t lo = 0, hi = 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    lo = max(lo, w[i] & 0x7FFFu);
-    hi = max(hi, (w[i] >> 16) & 0x7FFFu);
+  for (int i = 0; i < N; ++i) {
+    lo = max(lo, e[i] & 0x7FFFu);
+    hi = max(hi, (e[i] >> 16) & 0x7FFFu);
   }
   return max(lo, hi);
 }
 
 // The same with NaN elements left out (the exact path's absmax).
-__device__ __forceinline__ uint32_t lane_absmax_bits_nonnan(const uint4& a, const uint4& b) {
-  const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+template <int N>
+__device__ __forceinline__ uint32_t lane_absmax_bits_nonnan(const uint32_t (&e)[N]) {
   uint32_t m = 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t lo = w[i] & 0x7FFFu, hi = (w[i] >> 16) & 0x7FFFu;
+  for (int i = 0; i < N; ++i) {
+    const uint32_t lo = e[i] & 0x7FFFu, hi = (e[i] >> 16) & 0x7FFFu;
     m = max(m, lo > 0x7F80u ? 0u : lo);
     m = max(m, hi > 0x7F80u ? 0u : hi);
   }
   return m;
 }
 
-// Maximum over each group of 8 lanes (a scale block), in every lane of it.
-__device__ __forceinline__ uint32_t group8_max_u32(uint32_t k) {
+// Maximum over the lanes of a scale block (8 lanes of 16 elements or 16 lanes
+// of 8), in every lane of it.
+template <int LANES>
+__device__ __forceinline__ uint32_t block_max_u32(uint32_t k) {
+  static_assert(LANES == 8 || LANES == 16, "DPP rows");
+  if (LANES == 16) return row16_max_u32(k);
   k = max(k, dpp_u32<kDppQuad1032, 0xF>(k));
   k = max(k, dpp_u32<kDppQuad2301, 0xF>(k));
   return max(k, dpp_u32<kDppRowHalfMirror, 0xF>(k));
@@ -121,28 +125,35 @@ __device__ __forceinline__ uint32_t exact_pack4(float x0, float x1, float x2, fl
          (f32_to_e4m3_satfinite(x2 / s) << 16) | (f32_to_e4m3_satfinite(x3 / s) << 24);
 }
 
-// One pass of a wave: 16 elements per lane (a, b), 8 lanes per scale block;
+// One pass of a wave: 2N elements per lane, kBlk / 2N lanes per scale block;
 // the e4m3 codes and this lane's block scale (wave-uniform fast/exact branch).
-__device__ __forceinline__ void quantize_pass(const uint4& a, const uint4& b, uint4& out, float& s) {
-  const uint32_t m = group8_max_u32(lane_absmax_bits(a, b));
+template <int N>
+__device__ __forceinline__ void quantize_pass(const uint32_t (&e)[N], uint32_t (&out)[N / 2], float& s) {
+  constexpr int kLanes = kBlk / (2 * N);
+  const uint32_t m = block_max_u32<kLanes>(lane_absmax_bits(e));
   const bool odd = m > 0x7F7Fu || (m != 0u && m < kQTinyBf16);
-  const uint32_t e[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
   if (__ballot(odd) == 0) {
     const float amax = __uint_as_float(m << 16);
     s = amax > 0.0f ? amax / 448.0f : 1.0f;
     const float r = 1.0f / s;
-    out.x = fast_pack4(bf16_lo(e[0]), bf16_hi(e[0]), bf16_lo(e[1]), bf16_hi(e[1]), s, r);
-    out.y = fast_pack4(bf16_lo(e[2]), bf16_hi(e[2]), bf16_lo(e[3]), bf16_hi(e[3]), s, r);
-    out.z = fast_pack4(bf16_lo(e[4]), bf16_hi(e[4]), bf16_lo(e[5]), bf16_hi(e[5]), s, r);
-    out.w = fast_pack4(bf16_lo(e[6]), bf16_hi(e[6]), bf16_lo(e[7]), bf16_hi(e[7]), s, r);
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i)
+      out[i] = fast_pack4(bf16_lo(e[2 * i]), bf16_hi(e[2 * i]), bf16_lo(e[2 * i + 1]), bf16_hi(e[2 * i + 1]), s, r);
   } else {
-    const float amax = __uint_as_float(group8_max_u32(lane_absmax_bits_nonnan(a, b)) << 16);
+    const float amax = __uint_as_float(block_max_u32<kLanes>(lane_absmax_bits_nonnan(e)) << 16);
     s = amax > 0.0f ? amax / 448.0f : 1.0f;
-    out.x = exact_pack4(bf16_lo(e[0]), bf16_hi(e[0]), bf16_lo(e[1]), bf16_hi(e[1]), s);
-    out.y = exact_pack4(bf16_lo(e[2]), bf16_hi(e[2]), bf16_lo(e[3]), bf16_hi(e[3]), s);
-    out.z = exact_pack4(bf16_lo(e[4]), bf16_hi(e[4]), bf16_lo(e[5]), bf16_hi(e[5]), s);
-    out.w = exact_pack4(bf16_lo(e[6]), bf16_hi(e[6]), bf16_lo(e[7]), bf16_hi(e[7]), s);
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i)
+      out[i] = exact_pack4(bf16_lo(e[2 * i]), bf16_hi(e[2 * i]), bf16_lo(e[2 * i + 1]), bf16_hi(e[2 * i + 1]), s);
   }
+}
+
+// 16 elements of one lane (two 16-byte loads), 8 lanes per scale block.
+__device__ __forceinline__ void quantize_pass16(const uint4& a, const uint4& b, uint4& out, float& s) {
+  const uint32_t e[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  uint32_t o[4];
+  quantize_pass(e, o, s);
+  out = uint4{o[0], o[1], o[2], o[3]};
 }
 
 __global__ void __launch_bounds__(kQThreads)
@@ -166,7 +177,7 @@ quantize_hidden_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __restric
     for (int c = 0; c < kQPasses; ++c) {
       uint4 out;
       float s;
-      quantize_pass(raw[2 * c], raw[2 * c + 1], out, s);
+      quantize_pass16(raw[2 * c], raw[2 * c + 1], out, s);
       *(uint4*)(qrow + c * kQPass) = out;
       if ((lane & (kQLanesPerBlk - 1)) == 0) sc[c * (kQPass / kBlk) + lane / kQLanesPerBlk][w] = s;
     }
@@ -195,7 +206,7 @@ quantize_hidden_rows_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __re
   const uint4 a = *(const uint4*)src, b = *(const uint4*)(src + 8);
   uint4 out;
   float s;
-  quantize_pass(a, b, out, s);
+  quantize_pass16(a, b, out, s);
   *(uint4*)(q + (size_t)t * kH + c * kQPass + lane * kQLaneCols) = out;
   if ((lane & (kQLanesPerBlk - 1)) == 0) scale[(size_t)(c * (kQPass / kBlk) + lane / kQLanesPerBlk) * T + t] = s;
 }
@@ -215,33 +226,6 @@ constexpr int kQStreamPass = kWave * 8;            // 512 columns
 constexpr int kQStreamPasses = kQHalf / kQStreamPass;  // 7
 static_assert(kQStreamPasses * kQStreamPass == kQHalf && 16 * 8 == kBlk, "whole passes, 16 lanes per scale block");
 
-// One pass of a wave: 8 elements per lane, 16 lanes per scale block.
-__device__ __forceinline__ void quantize_pass8(const v4i& a, uint2& out, float& s) {
-  const uint32_t e[4] = {(uint32_t)a[0], (uint32_t)a[1], (uint32_t)a[2], (uint32_t)a[3]};
-  uint32_t m = 0, ok = 0;  // largest magnitude (bf16 bits), with and without NaN elements
-#pragma unroll
-  for (int i = 0; i < 4; ++i) m = max(m, max(e[i] & 0x7FFFu, (e[i] >> 16) & 0x7FFFu));
-  m = row16_max_u32(m);
-  const bool odd = m > 0x7F7Fu || (m != 0u && m < kQTinyBf16);
-  if (__ballot(odd) == 0) {
-    const float amax = __uint_as_float(m << 16);
-    s = amax > 0.0f ? amax / 448.0f : 1.0f;
-    const float r = 1.0f / s;
-    out.x = fast_pack4(bf16_lo(e[0]), bf16_hi(e[0]), bf16_lo(e[1]), bf16_hi(e[1]), s, r);
-    out.y = fast_pack4(bf16_lo(e[2]), bf16_hi(e[2]), bf16_lo(e[3]), bf16_hi(e[3]), s, r);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t lo = e[i] & 0x7FFFu, hi = (e[i] >> 16) & 0x7FFFu;
-      ok = max(ok, max(lo > 0x7F80u ? 0u : lo, hi > 0x7F80u ? 0u : hi));
-    }
-    const float amax = __uint_as_float(row16_max_u32(ok) << 16);
-    s = amax > 0.0f ? amax / 448.0f : 1.0f;
-    out.x = exact_pack4(bf16_lo(e[0]), bf16_hi(e[0]), bf16_lo(e[1]), bf16_hi(e[1]), s);
-    out.y = exact_pack4(bf16_lo(e[2]), bf16_hi(e[2]), bf16_lo(e[3]), bf16_hi(e[3]), s);
-  }
-}
-
 __global__ void __launch_bounds__(kWave)
 quantize_hidden_stream_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __restrict__ q,
                               float* __restrict__ scale) {
@@ -254,10 +238,11 @@ quantize_hidden_stream_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __
   for (int c = 0; c < kQStreamPasses; ++c) raw[c] = __builtin_nontemporal_load((const v4i*)(src + c * kQStreamPass));
 #pragma unroll
   for (int c = 0; c < kQStreamPasses; ++c) {
-    uint2 out;
+    const uint32_t e[4] = {(uint32_t)raw[c][0], (uint32_t)raw[c][1], (uint32_t)raw[c][2], (uint32_t)raw[c][3]};
+    uint32_t out[2];
     float s;
-    quantize_pass8(raw[c], out, s);
-    *(uint2*)(dst + c * kQStreamPass) = out;
+    quantize_pass(e, out, s);
+    *(uint2*)(dst + c * kQStreamPass) = uint2{out[0], out[1]};
     if ((lane & 15) == 0) scale[(size_t)((c0 + c * kQStreamPass) / kBlk + (lane >> 4)) * T + t] = s;
   }
 }
