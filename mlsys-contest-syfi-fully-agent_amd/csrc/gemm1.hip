@@ -404,13 +404,21 @@ gemm1_stream_kernel(const uint8_t* __restrict__ hs, const float* __restrict__ hs
 //     products), acc += P * (a_scale[row] * w_scale[n/128]).
 // ---------------------------------------------------------------------------
 // Kernel choice by T: the tiled kernel below kGemm1WideMinTokens, the wide tiles
-// from it on.  Both give the same output bits.  Below it most experts hold few
-// rows and 16 column tiles of each leave the 256 one-workgroup CUs unevenly
-// filled (20 experts: 1.25 rounds), where the tiled kernel's 32 on 512 slots do
-// not.  Interleaved A/B, GEMM1 us, tiled -> wide: prefill routing T = 200 101 ->
-// 117, 512 106 -> 118, 700 121 -> 133, 900 131 -> 135, 1024 152 -> 138, 1280
-// 152 -> 137, 1500 170 -> 149; four hot experts T = 1024 230 -> 217 (and 512
-// 177 -> 139, but T alone does not tell them from the others).
+// from it on.  Both give the same output bits.  Where most experts hold few
+// rows, 16 column tiles of each leave the 256 one-workgroup CUs unevenly filled
+// (20 experts: 1.25 rounds), which the tiled kernel's 32 on 512 slots do not.
+// What decides is rows per expert, which the host does not know and which vary
+// with the input (uniform routing, T = 1024: 404 to 1,549 pairs over eight
+// seeds).  Interleaved A/B, GEMM1 us with the events around it, geometric means
+// over eight inputs, tiled -> wide:
+//   uniform routing   T = 333 102 -> 111, 512 116 -> 121, 640 123 -> 125, 800
+//     127 -> 128, 900 132 -> 129, 1000 139 -> 131, 1024 140 -> 131, 1280 148 ->
+//     136, 1536 155 -> 139, 2000 180 -> 155;
+//   four hot experts  T = 333 123 -> 112, 512 159 -> 119, 800 202 -> 173, 1000
+//     228 -> 210, 1024 228 -> 210, 1536 310 -> 259.
+// By it inputs of few pairs lose: T = 1024 404 pairs 108 -> 111, 911 pairs 131 ->
+// 140, T = 1280 726 pairs 133 -> 137, T = 1536 580 pairs 107 -> 112; and hot
+// experts at smaller T, as above.
 constexpr int kGemm1WideMinTokens = 1024;
 static_assert(kGemm1WideMinTokens <= kEveryTokenFuseMinTokens, "only the wide kernel folds routing weights in");
 
@@ -770,7 +778,10 @@ hipError_t launch_gemm1_tiled(const uint8_t* hs, const float* hs_scale, int T, c
 //     flight, and all tall tiles before all short ones, took GEMM1 from 272 to
 //     236 us at T = 4096 (prefill routing), 217 to 187 at T = 3000, 195 to 174 at
 //     T = 2000, 574 to 539 at T = 14107; hot experts T = 1451 294 -> 275, 8192
-//     1,094 -> 1,077 (same bits).  64-row tiles on top gained nothing.
+//     1,094 -> 1,077 (same bits; one input each, prefill routing of seed 1).
+//     Over eight inputs: T = 2000 191 -> 155, 3072 217 -> 184, four hot experts
+//     1451 286 -> 251, 3072 471 -> 454, where one input whose hot rows fill whole
+//     rounds of tall tiles lost, 404 -> 430.  64-row tiles on top gained nothing.
 // Common to both:
 //   * the workgroup's 128 gate columns (and its 128 up columns) are one
 //     128-column weight scale block, so one gate and one up scale per K block;

@@ -384,12 +384,21 @@ struct G2Tiled {
 //     freeing its slot at once for the stage two ahead;
 //   * e4m3 -> bf16 conversions run once per W2 value (the 64 x 256 tile's two
 //     row waves each convert all of a column's).
-// Interleaved A/B, GEMM2 us (64 x 256 tiles only -> with low tiles): prefill
-// routing T = 65 48 -> 40, 333 102 -> 79, 512 97 -> 76, 700 104 -> 93, 1024
-// 107 -> 102, 2000 150 -> 148, 3000 195 -> 193; hot experts T = 128 80 -> 65,
-// 1451 335 -> 328.  An extra row block (33 to 64 rows, act rows 32 KB per 128
-// K) gained nothing, nor did 48-column waves; low tiles ahead of the others
-// lost 5-8 us at T = 128 to 512 (they are the shorter ones).
+// Interleaved A/B, GEMM2 us with the events around it, geometric means over six
+// to eight inputs (64 x 256 tiles only -> with low tiles): uniform routing T = 65
+// 40 -> 34, 256 64 -> 53, 333 60 -> 53, 512 81 -> 68, 720 83 -> 76, 1024 93 -> 86,
+// 2000 132 -> 126, 3072 174 -> 171; four hot experts T = 65 58 -> 46, 150 78 -> 62,
+// 256 92 -> 89, 512 138 -> 139, 800 201 -> 196, 1024 235 -> 223, 1451 324 -> 319.
+// From T = 300 to 720 some inputs with four hot experts lose (512, 32 full row
+// tiles and 18 low experts: 141 -> 156): the full tiles, bound by their MFMAs,
+// and the low ones, bound by the W2 stream, no longer run side by side.  Low
+// tiles dealt between the full ones where these are more than run at once (512)
+// gained 3 % of GEMM2 with 512 to 640 full tiles and nothing on average beyond.
+// An extra row block (33 to 64 rows, act rows 32 KB per 128 K) gained nothing,
+// nor did 48-column waves; low tiles ahead of the others lost 5-8 us at T = 128
+// to 512 (they are the shorter ones).  Four-wave tiles of 128 columns, four to a
+// CU, at T = 9 to 32: 10 to 13 experts with rows 35 -> 31 us, 5 or 6 experts
+// 18.6 -> 20.0, 14 or more no gain.
 // ---------------------------------------------------------------------------
 template <int RB_>
 struct G2Low {
@@ -558,8 +567,8 @@ __device__ __forceinline__ void gemm2_low_tile(char* lds, const uint16_t* __rest
   }
 }
 
-// Low tiles up to this T.  T = 3000 gains 1 % of GEMM2, T = 4096 ties (255 / 252
-// us); at T = 8192 and 14107 (uniform routing, many rounds of full tiles) the
+// Low tiles up to this T.  T = 3072 gains 1 to 2 % of GEMM2, T = 4096 ties (255 /
+// 252 us); at T = 8192 and 14107 (uniform routing, many rounds of full tiles) the
 // few low tiles at the end of the launch run alone, bound by latency: 405 ->
 // 407, 746 -> 758 us.
 constexpr int kG2LowMaxTokens = 3072;

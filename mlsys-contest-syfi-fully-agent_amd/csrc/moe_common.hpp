@@ -37,12 +37,19 @@ static_assert(kMaxTokens * kH <= (int64_t)1 << 32, "token row offsets fit in 32 
 // Largest T for which GEMM2 also performs the weighted combine: its rows
 // never reach the workspace, and no combine pass runs.  Each of its workgroups
 // loads every expert's act rows (16-row MFMA operands straight from L2, ~4 us
-// a job of more than 8 rows); beyond 8 tokens the tiled kernel's low tiles and
-// a combine pass are faster or tie.  Layer us, fused -> tiled + combine: four
-// hot experts T = 16 99 -> 89, 17 111 -> 93, 51 186 -> 134, 64 202 -> 142, two
-// T = 12 83 -> 76, 8 73.3 -> 72.0, 4 55 -> 58; uniform routing T = 64 157 ->
-// 137, 48 133 -> 124, 33 125 -> 119, 24 113 -> 111, 16 85.3 -> 85.3, 7 64.7 ->
-// 66.8.
+// a job of more than 8 rows); the tiled kernel's low tiles read them once per
+// 256 columns, but its rows need a combine pass (~2 us and a launch).  What
+// decides is rows per expert, which the host does not know.  Layer us, fused ->
+// tiled + combine, geometric means over five to seven inputs:
+//   uniform routing  T = 4 39 -> 44, 8 40 -> 46, 9 52 -> 54, 12 59 -> 62,
+//     16 71 -> 72, 20 78 -> 78, 32 94 -> 94, 48 115 -> 108, 64 128 -> 120;
+//   two hot experts  T = 4 42 -> 46, 8 56 -> 57, 9 66 -> 63, 12 75 -> 69,
+//     16 92 -> 85, 32 134 -> 120, 64 177 -> 144;
+//   four             T = 4 47 -> 49, 8 62 -> 60, 9 70 -> 65, 12 77 -> 69,
+//     16 88 -> 78, 32 134 -> 110, 64 191 -> 131.
+// The line lies where two hot experts change sides.  Uniform routing loses 1
+// to 3 us from T = 9 to 16 by it (an input of three pairs 34 -> 40), four hot
+// experts 2 us at T = 8.
 constexpr int kGemm2StreamMaxTokens = 8;
 // From this T on, experts that every token selects are summed inside GEMM2
 // (every_token_experts).  Below it the fused tiles (T / 64 row tiles x 28

@@ -10,10 +10,9 @@
 // Design (gfx950): HBM-bound (reads 2 B and writes 1 B per element), so the
 // arithmetic per element has to stay under the memory time.  Up to T = 2048
 // one workgroup per token row, wave p quantising pass p (7 waves per row, so
-// that enough loads are in flight at small T).  From T = 5120, where the rows
-// outgrow the caches, half a row per wave with nontemporal loads
-// (quantize_hidden_stream_kernel).  Between, one wave per token
-// row, four rows per workgroup (T/4 workgroups: 1024 at T = 4096).  A
+// that enough loads are in flight at small T).  From T = 5120 half a row per
+// wave with nontemporal loads (quantize_hidden_stream_kernel).  Between, one wave
+// per token row, four rows per workgroup (T/4 workgroups: 1024 at T = 4096).  A
 // wave issues all 14 row loads (16 B per lane each) before any arithmetic, so
 // a token has its whole 14 KB row in flight at once; each of the 7 passes
 // then covers 1024 columns = 8 scale blocks, 8 lanes per block and 16
@@ -215,11 +214,17 @@ quantize_hidden_rows_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __re
 // elements a pass (16 lanes per scale block), so each load instruction covers
 // 1 KB of contiguous bytes (16 elements per lane would touch every line
 // twice), and the rows, read once, are loaded nontemporally.  Same arithmetic,
-// same bits.  us, one wave per row with temporal loads -> this: T = 14107 58.9
-// -> 54.5, 10000 42.4 -> 37.7 (5.8 TB/s), 8192 35.7 -> 31.6, 5632 25.6 -> 23.5,
-// 5120 22.8 -> 22.1; at T = 4608 a tie, and below it the nontemporal loads lose
-// (4096 17.4 -> 18.4: there the rows are still cached).  Nontemporal stores
-// gained another 0-4 % but would send the layer's input past the caches.
+// same bits.  It fetches what the rows hold (T = 8192 117.6 of 117.4 MB).  us, one
+// wave per row with temporal loads -> this, where rows and outputs of the last
+// calls push each other out of the caches: T = 14107 58.5 -> 53.6, 10000 42.5 ->
+// 37.7 (5.8 TB/s), 8192 36.1 -> 31.5, 7000 30.9 -> 27.5, 5632 25.4 -> 23.5, 5120
+// 22.2 -> 22.0; below it the nontemporal loads lose (4096 17.4 -> 18.4).  Rows
+// that the step before has just written, into an output that every call
+// reuses, are partly in the caches, where nontemporal loads gain less or lose:
+// 5120 22.6 -> 25.2, 7000 29.4 -> 31.0, 8192 33.5 -> 34.6, 10000 40.4 -> 41.0,
+// 14107 60.0 -> 55.6.  This layout with temporal loads keeps the old kernel's
+// times in both (8192 38.2 and 33.3).  Nontemporal stores gained another 0-4 %
+// but would send the layer's input past the caches.
 constexpr int kQStreamMinTokens = 5120;
 constexpr int kQHalf = kH / 2;                     // columns per wave
 constexpr int kQStreamPass = kWave * 8;            // 512 columns
