@@ -16,8 +16,9 @@ namespace {
 // ---- scratch of the no-allocation entry point -----------------------------
 // moe_fp8_ds_run_noalloc keeps its intermediates in this file-scope device
 // array instead of a caller workspace: the layer's workspace layout for
-// MOE_FP8_DS_NOALLOC_MAX_TOKENS tokens.  Each device the library runs on
-// holds its own copy (loaded with the code object) until the process ends.
+// MOE_FP8_DS_NOALLOC_MAX_TOKENS tokens, 19 MB: 4.2 MB and the GEMM2 rows of 512
+// pairs (from T = 9 the combine is a pass of its own).  Each device the library
+// runs on holds its own copy (loaded with the code object) until the process ends.
 // In host code `scratch` only names the symbol; its device address comes from
 // hipGetSymbolAddress, once per device (noalloc_scratch).
 constexpr size_t kNoAllocScratchBytes = moe::make_layout(MOE_FP8_DS_NOALLOC_MAX_TOKENS).total;
