@@ -222,9 +222,10 @@ quantize_hidden_rows_kernel(const uint16_t* __restrict__ x, int T, uint8_t* __re
 // that the step before has just written, into an output that every call
 // reuses, are partly in the caches, where nontemporal loads gain less or lose:
 // 5120 22.6 -> 25.2, 7000 29.4 -> 31.0, 8192 33.5 -> 34.6, 10000 40.4 -> 41.0,
-// 14107 60.0 -> 55.6.  This layout with temporal loads keeps the old kernel's
-// times in both (8192 38.2 and 33.3).  Nontemporal stores gained another 0-4 %
-// but would send the layer's input past the caches.
+// 14107 60.0 -> 55.6 (one kernel timed as both sides there differs by 2 %).  This
+// layout with temporal loads keeps the old kernel's times in both (8192 38.2 and
+// 33.3).  Nontemporal stores gained another 0-4 % but would send the layer's
+// input past the caches.
 constexpr int kQStreamMinTokens = 5120;
 constexpr int kQHalf = kH / 2;                     // columns per wave
 constexpr int kQStreamPass = kWave * 8;            // 512 columns
